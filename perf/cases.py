@@ -33,19 +33,19 @@ VEL_SCALE = 0.5
 def listed():
     return [
         # a room with a few hundred people, drawn every frame: launches and latency
-        crowd("room, drawn every step", 30.0, 6, 12, 500, read_every=True),
+        crowd("room", 30.0, 6, 12, 500, read_every=True),
         # c0 of the benchmark: 200 m, 40 obstacles, 5,000 agents
         crowd("c0", 100.0, 40, 15, 5000),
         # c0 with the reference's literal parameters, drawn every step
-        crowd("c0, reference parameters", 100.0, 40, 15, 5000, k=5, reference=True, read_every=True),
+        crowd("c0 reference", 100.0, 40, 15, 5000, k=5, reference=True, read_every=True),
         # a town square between the benchmark's sizes; k off the defaults, agents off every power of two
-        crowd("town, k 7", 350.0, 197, 20, 37411, k=7),
+        crowd("town", 350.0, 197, 20, 37411, k=7),
         # c1: 1000 m, 400 obstacles, 100,000 agents
         crowd("c1", 500.0, 400, 25, 100000),
         # c2: a million agents in two opposing flows, jammed in the barrier's gaps
-        flows("c2, jam", 950000),
+        flows("c2 jam", 950000),
         # the same with the learned proposal in front of the LP
-        flows("c2, jam, learned", 950000, learned=True),
+        flows("c2 jam learned", 950000, learned=True),
         # c4 in small: independent environments advanced by one handle
         {"name": "24 environments", "kind": "batch", "envs": 24, "k": 10, "steps": 20, "prerun": 20, "map": 5},
         # the network on device buffers, the largest call it takes
