@@ -36,6 +36,7 @@ hipError_t launch_mark_dead(const int* ids, int n, const int* pos_of, const floa
                             const unsigned long long* acc, hipStream_t st);
 hipError_t launch_attr_knn(const DevState& s, int block, int mode, int oslots, hipStream_t st, hipEvent_t mid);
 hipError_t launch_orca(const DevState& s, int maxo, int mode, int oslots, int n_cu, hipStream_t st, hipEvent_t mid);
+hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st, hipEvent_t mid);
 hipError_t launch_features(const DevState& s, hipStream_t st);
 hipError_t launch_export_nbrs(const DevState& s, int* out, int* out_cnt, hipStream_t st);
 hipError_t launch_spawn_scatter(int n, const int* ids, const float2* start, const float* rad, const float* spd,
@@ -264,7 +265,7 @@ struct ecm_sim {
     // recaptured when anything they were captured with changes
     struct GraphKey {
         DevState d;
-        int maxo, mode, oslots, knn_block, n_cu;
+        int maxo, mode, oslots, knn_block, n_cu, row;
         float theta;
         const void* frags;
         const void* pbias;
@@ -276,6 +277,7 @@ struct ecm_sim {
         hipGraphExec_t exec[2] = {nullptr, nullptr};
     };
     bool use_graph = false;
+    bool row_step = false;                      // 16 lanes per agent (row_step_rule)
     StepGraph graphs[2][2];                     // [parity][entry from the sorted outputs]
     std::string graph_error;
     std::vector<int> h_replans;
@@ -1550,6 +1552,17 @@ static int prepare_step(ecm_sim* s, DevState* out) {
     return 0;
 }
 
+// 16 lanes per agent (row_kernels.h) for the plain step of a small crowd in
+// the default launch shape; other shapes say how agents are laid out.
+static constexpr int kRowAgents = 40000;
+
+static void row_step_rule(ecm_sim* s, int mode) {
+    // a crowd near the limit keeps the form it has: changing it captures the
+    // step graphs anew
+    const int limit = s->row_step ? kRowAgents + kRowAgents / 4 : kRowAgents;
+    s->row_step = mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2 && s->num_agents <= limit;
+}
+
 static int step_mode(const ecm_sim* s) { return s->log_mlp ? 1 : (s->mlp ? 2 : 0); }
 
 // The device operations of one step, in stream order, in two halves: up to
@@ -1562,6 +1575,10 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
         // into the totals and clears them for this step
         HIPCHK(launch_grid_build(d, s->bsum.p, s->stream));
         if (s->timing) HIPCHK(hipEventRecord(s->ev[1], s->stream));
+        if (s->row_step) {
+            HIPCHK(launch_row_step(d, s->maxo, s->n_cu, s->stream, s->timing ? s->ev[6] : nullptr));
+            return 0;
+        }
         // the plain step's main ORCA pass may run inside this kernel (k 5
         // and 10): its events are published once both are done
         HIPCHK(launch_attr_knn(d, s->tune.knn_block, mode, s->tune.orca_obst_slots, s->stream,
@@ -1579,7 +1596,12 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
                                      s->mlp_theta, s->mlp_mask.p, nullptr, nullptr, s->mlp->n_cu, s->stream));
     }
     if (s->timing) HIPCHK(hipEventRecord(s->ev[3], s->stream));
-    HIPCHK(launch_orca(d, s->maxo, mode, s->tune.orca_obst_slots, s->n_cu, s->stream, s->timing ? s->ev[5] : nullptr));
+    if (s->row_step) {
+        if (s->timing) HIPCHK(hipEventRecord(s->ev[5], s->stream));
+    } else {
+        HIPCHK(launch_orca(d, s->maxo, mode, s->tune.orca_obst_slots, s->n_cu, s->stream,
+                           s->timing ? s->ev[5] : nullptr));
+    }
     if (s->timing) HIPCHK(hipEventRecord(s->ev[4], s->stream));
     return 0;
 }
@@ -1631,6 +1653,7 @@ static int ensure_step_graph(ecm_sim* s, const DevState& d, int mode) {
     key.frags = mode == 2 ? (const void*)s->mlp->frags.p : nullptr;
     key.pbias = mode == 2 ? (const void*)s->mlp->pbias.p : nullptr;
     key.n_cu = mode == 2 ? s->mlp->n_cu : 0;
+    key.row = s->row_step ? 1 : 0;
     ecm_sim::StepGraph& g = s->graphs[s->cur][d.sorted_in];
     if (g.valid && std::memcmp(&g.key, &key, sizeof(key)) == 0) return 0;
     if (int rc = settle(s)) return rc;      // an earlier launch of g may still run
@@ -1669,6 +1692,7 @@ static int step_once(ecm_sim* s) {
     int rc = prepare_step(s, &d);
     if (rc) return rc;
     const int mode = step_mode(s);
+    row_step_rule(s, mode);
     bool graph = false;
     if (s->use_graph && !s->timing) {
         rc = ensure_step_graph(s, d, mode);

@@ -782,6 +782,25 @@ static constexpr int kKnnBuf = 16;
 static constexpr float kKnnWalkCells = 6.0f;
 static constexpr int kKnnRanges = 4;
 
+// DestroyAgent for sorted agent t: the slot keeps the state it is destroyed
+// with: step-start position and velocity, this step's attraction point, the
+// previous step's preferred and ORCA velocities (already there after a step
+// that started from the slot arrays).  Appends the event and fences it.
+__device__ __forceinline__ void retire_agent(const DevState& s, int t, int id, V2 pos, float4 sv, V2 attr) {
+    s.pos_in[id] = make_float2(pos.x, pos.y);
+    s.vel_in[id] = make_float2(sv.x, sv.y);
+    s.attraction[id] = make_float2(attr.x, attr.y);
+    const int qp = s.prev_of[t];
+    if (s.sorted_in && qp >= 0) {
+        s.pref_vel[id] = s.pref_vel_s_old[qp];
+        if (s.v_orca) s.v_orca[id] = s.v_orca_s_old[qp];
+    }
+    s.active[id] = 0;
+    const uint32_t q = atomicAdd(s.events_n, 1u);
+    s.events[q] = make_int4(id, 0, 0, -1);
+    __threadfence();
+}
+
 // One sorted agent's goal check, attraction point and steering (with the
 // destroy or replan request they may make).  Returns whether it appended an
 // event, after fencing it device-wide.
@@ -823,22 +842,7 @@ __device__ __forceinline__ bool attr_agent(const DevState& s) {
     if (fb) atomicAdd(&s.stats[2], 1u);
     s.dead_s[t] = alive ? 0 : 1;
     if (!alive) {
-        // the slot keeps the state it is destroyed with: step-start position
-        // and velocity, this step's attraction point, the previous step's
-        // preferred and ORCA velocities (already there after a step that
-        // started from the slot arrays)
-        s.pos_in[id] = make_float2(pos.x, pos.y);
-        s.vel_in[id] = make_float2(sv.x, sv.y);
-        s.attraction[id] = make_float2(attr.x, attr.y);
-        const int qp = s.prev_of[t];
-        if (s.sorted_in && qp >= 0) {
-            s.pref_vel[id] = s.pref_vel_s_old[qp];
-            if (s.v_orca) s.v_orca[id] = s.v_orca_s_old[qp];
-        }
-        s.active[id] = 0;                                   // DestroyAgent
-        uint32_t q = atomicAdd(s.events_n, 1u);
-        s.events[q] = make_int4(id, 0, 0, -1);
-        __threadfence();
+        retire_agent(s, t, id, pos, sv, attr);
         return true;
     }
     // ApplySteeringForce (Simulator.cpp:638-657)
@@ -1999,6 +2003,11 @@ __global__ void k_export_nbrs(DevState s, int* out, int* out_cnt) {
     out_cnt[id] = cnt;
 }
 
+// Obstacle constraints the main pass of the default launch shape holds; more
+// of them count as overflow in the statistics.
+static constexpr int kRowStatObst = 4;
+#include "row_kernels.h"
+
 // ------------------------------------------------------------- launchers
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 static inline int round8(int n) { return (n + 7) & ~7; }
@@ -2107,6 +2116,20 @@ static void launch_orca_k(const DevState& s, int maxo, int mode, int oslots, int
         hipLaunchKernelGGL((k_lp3d_reg<K, kLp3dRegObst>), gr, br, 0, st, s);
         hipLaunchKernelGGL((k_lp3d_wide<K>), gq, b, (size_t)(maxo + 2 * K) * sizeof(float4), st, s, maxo);
     }
+}
+
+// The passes with 16 lanes per agent (row_kernels.h): the whole rest of the
+// plain step after the grid build.  Grids of at most 32 wavefronts per CU,
+// strided, so that spare slots of a large pool cost nothing.
+hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st, hipEvent_t mid) {
+    const int cap = std::max(1, n_cu) * 32;
+    const dim3 ga(std::min(round8(cdiv(s.n_slots, 16)), round8(cap / 4)));
+    hipLaunchKernelGGL(k_attr_row, ga, dim3(256), 0, st, s);
+    if (mid) (void)hipEventRecord(mid, st);
+    const int row_f4 = std::max(maxo, kRowLdsBytes / 16);
+    hipLaunchKernelGGL(k_row_step, dim3(std::min(round8(cdiv(s.n_slots, 4)), round8(cap))), dim3(64),
+                       (size_t)row_f4 * 4 * sizeof(float4), st, s, maxo, row_f4);
+    return hipGetLastError();
 }
 
 // `mid`, when not null, is recorded between the attraction pass and the
