@@ -148,22 +148,16 @@ __device__ __forceinline__ bool row_irm(const EnvDesc& s, V2 pos, const float2* 
     return success;
 }
 
-// attr_agent for the agent at sorted position t, with 16 lanes.  Returns
-// whether this lane appended an event, after fencing it device-wide.
-__device__ __forceinline__ bool row_attr_agent(const DevState& s, int t, int l) {
-    const float4 pr = s.sorted_pr[t];
-    const float4 sv = s.sorted_v[t];
-    const int2 pc = s.path_s[t];
-    const float2 a0 = s.attr_s[t];
-    const int id = __float_as_int(pr.w);
-    const V2 pos = mk(pr.x, pr.y);
-    const EnvDesc& E = env_of_sorted(s, sv);
-    const int np = pc.y;
-    const float2* path = s.path_pts + pc.x;
+// attr_agent with 16 lanes.
+__device__ __forceinline__ void row_attr_agent(const DevState& s, int t, int l, const AttrIn& in) {
+    const V2 pos = mk(in.pr.x, in.pr.y);
+    const EnvDesc& E = env_of_sorted(s, in.sv);
+    const int np = in.pc.y;
+    const float2* path = s.path_pts + in.pc.x;
     const float2 gg = path[np - 1];
     const float gx = pos.x - gg.x, gy = pos.y - gg.y;
     const float dGoal = gx * gx + gy * gy;
-    V2 attr = mk(a0.x, a0.y);
+    V2 attr = mk(in.a0.x, in.a0.y);
     bool alive = true, event = false;
     uint32_t fb = 0;
     if (dGoal < s.arrival_r2) {
@@ -174,32 +168,46 @@ __device__ __forceinline__ bool row_attr_agent(const DevState& s, int t, int l) 
         if (row_irm(E, pos, path, np, l, ap, fb)) attr = ap;
         else event = true;
     }
-    if (l != 0) return false;
+    if (l != 0) return;
     if (event) {
         // UpdatePath(e, currentPosition, goal) with the step-start position
         const uint32_t q = atomicAdd(s.events_n, 1u);
-        s.events[q] = make_int4(id, __float_as_int(pos.x), __float_as_int(pos.y), t);
+        s.events[q] = make_int4(__float_as_int(in.pr.w), __float_as_int(pos.x), __float_as_int(pos.y), t);
     }
     s.attr_s[t] = make_float2(attr.x, attr.y);
     if (fb) atomicAdd(&s.stats[2], 1u);
     s.dead_s[t] = alive ? 0 : 1;
     if (!alive) {
-        retire_agent(s, t, id, pos, sv, attr);
-        return true;
+        retire_agent(s, in, attr);
+        return;
     }
-    const V2 des = normalize(attr - pos) * sv.z;
+    const V2 des = normalize(attr - pos) * in.sv.z;
     s.pref_vel_s[t] = make_float2(des.x, des.y);
     if (event) __threadfence();
-    return event;
 }
 
-// k_attr with 16 lanes per agent.
+// k_attr and k_scatter_attr with 16 lanes per agent: 14 -> 10 us at 500 agents
+// and 18 -> 13 at 5,000; at 37,000 40 instead of 21 (four times the
+// wavefronts wait on the same loads), so larger crowds keep one lane.
 __global__ __launch_bounds__(256) void k_attr_row(DevState s) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) s.acc[15] = 0;   // the grid build has used it
     const int n_active = (int)s.cell_start[s.n_keys];
     const int per = blockDim.x / kRow, l = threadIdx.x & (kRow - 1);
     for (int t = xcd_block() * per + (int)threadIdx.x / kRow; t < n_active; t += gridDim.x * per)
-        row_attr_agent(s, t, l);
+        row_attr_agent(s, t, l, attr_in(s, t));
+    publish_if_last(s);
+}
+
+__global__ __launch_bounds__(256) void k_scatter_attr_row(DevState s) {
+    __shared__ uint32_t top[kTopMax];
+    const Starts S = scatter_starts(s, top);
+    const int n_old = (int)(uint32_t)s.acc[14], n = n_old + (int)(uint32_t)s.acc[15];
+    const int per = blockDim.x / kRow, l = threadIdx.x & (kRow - 1);
+    for (int t = xcd_block() * per + (int)threadIdx.x / kRow; t < n; t += gridDim.x * per) {
+        const uint32_t m = s.key[t];
+        if (m == kInvalidKey) continue;
+        const int slot = (int)(S.at(m) + s.rank[t]);
+        row_attr_agent(s, slot, l, scatter_agent(s, t, n_old, slot, l == 0));
+    }
     publish_if_last(s);
 }
 

@@ -29,14 +29,14 @@
 #include <vector>
 
 namespace ecm {
-hipError_t launch_grid_build(const DevState& s, uint32_t* bsum, hipStream_t st);
+hipError_t launch_grid_attr(const DevState& s, bool row, int n_cu, hipStream_t st, hipEvent_t mid);
 hipError_t launch_unsort(const DevState& s, hipStream_t st);
 hipError_t launch_unsort_pos(const DevState& s, hipStream_t st);
 hipError_t launch_mark_dead(const int* ids, int n, const int* pos_of, const float4* sorted_pr_old, uint8_t* dead_old,
                             const unsigned long long* acc, hipStream_t st);
-hipError_t launch_attr_knn(const DevState& s, int block, int mode, int oslots, hipStream_t st, hipEvent_t mid);
+hipError_t launch_knn(const DevState& s, int block, int mode, int oslots, hipStream_t st);
 hipError_t launch_orca(const DevState& s, int maxo, int mode, int oslots, int n_cu, hipStream_t st, hipEvent_t mid);
-hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st, hipEvent_t mid);
+hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st);
 hipError_t launch_features(const DevState& s, hipStream_t st);
 hipError_t launch_export_nbrs(const DevState& s, int* out, int* out_cnt, hipStream_t st);
 hipError_t launch_spawn_scatter(int n, const int* ids, const float2* start, const float* rad, const float* spd,
@@ -165,7 +165,7 @@ struct ecm_sim {
     int cur = 0;
 
     // agent grid
-    DBuf<uint32_t> key, rank, cell_count, cell_start, bsum;
+    DBuf<uint32_t> key, rank, cell_count, cell_local, cell_start, bsum;
     // sorted state by step parity: this step's [cur], the last step's [cur^1]
     DBuf<float4> sorted_pr[2], sorted_v[2];
     DBuf<float2> attr_s[2], pos_s[2], vel_s[2];
@@ -277,7 +277,7 @@ struct ecm_sim {
         hipGraphExec_t exec[2] = {nullptr, nullptr};
     };
     bool use_graph = false;
-    bool row_step = false;                      // 16 lanes per agent (row_step_rule)
+    bool row_step = false, row_attr = false;    // 16 lanes per agent (row_rule)
     StepGraph graphs[2][2];                     // [parity][entry from the sorted outputs]
     std::string graph_error;
     std::vector<int> h_replans;
@@ -318,7 +318,7 @@ static void free_all(ecm_sim* s) {
     for (int b = 0; b < 2; ++b) { s->pref_vel_s[b].release(); s->v_orca_s[b].release(); }
     s->radius.release(); s->pref_speed.release(); s->active.release();
     s->path_off.release(); s->path_cnt.release(); s->path_pool.release();
-    s->key.release(); s->rank.release(); s->cell_count.release(); s->cell_start.release(); s->bsum.release();
+    s->key.release(); s->rank.release(); s->cell_count.release(); s->cell_local.release(); s->cell_start.release(); s->bsum.release();
     for (int b = 0; b < 2; ++b) { s->nbr[b].release(); s->nbr_cnt[b].release(); }
     s->fwd.release(); s->prev_of.release(); s->pos_of.release();
     s->new_ids.release(); s->dead_ids.release();
@@ -1277,11 +1277,14 @@ static int ensure_agent_grid(ecm_sim* s) {
     }
     if (base >= 0xffffffffull) return fail(ECM_E_STATE, "agent grids of the environments exceed 2^32 cells");
     const size_t G = (size_t)base;
-    rc = s->cell_count.alloc(G);
+    // the scan works on whole blocks of kScanCells counts
+    const size_t GP = (G + kScanCells - 1) / kScanCells * kScanCells;
+    rc = s->cell_count.alloc(GP);
+    if (!rc) rc = s->cell_local.alloc(GP);
     if (!rc) rc = s->cell_start.alloc(G + 1);
-    if (!rc) rc = s->bsum.alloc((G + 1023) / 1024 + 1);
+    if (!rc) rc = s->bsum.alloc(GP / kScanCells);
     if (rc) return rc;
-    rc = zero_dev(s->cell_count.p, G * sizeof(uint32_t), s->stream);
+    rc = zero_dev(s->cell_count.p, GP * sizeof(uint32_t), s->stream);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(s->stream));
     s->n_keys = (uint32_t)G;
@@ -1350,6 +1353,7 @@ static DevState make_state(ecm_sim* s) {
     d.agent_env = s->envs.size() > 1 ? s->agent_env.p : nullptr;
     d.n_keys = s->n_keys;
     d.key = s->key.p; d.rank = s->rank.p; d.cell_count = s->cell_count.p; d.cell_start = s->cell_start.p;
+    d.cell_local = s->cell_local.p; d.bsum = s->bsum.p;
     d.sorted_pr = s->sorted_pr[s->cur].p; d.sorted_v = s->sorted_v[s->cur].p;
     d.nbr = s->nbr[s->cur].p; d.nbr_cnt = s->nbr_cnt[s->cur].p;
     d.nbr_prev = s->nbr[s->cur ^ 1].p; d.nbr_cnt_prev = s->nbr_cnt[s->cur ^ 1].p;
@@ -1554,13 +1558,15 @@ static int prepare_step(ecm_sim* s, DevState* out) {
 
 // 16 lanes per agent (row_kernels.h) for the plain step of a small crowd in
 // the default launch shape; other shapes say how agents are laid out.
-static constexpr int kRowAgents = 40000;
+static constexpr int kRowAgents = 40000, kRowAttrAgents = 16000;
 
-static void row_step_rule(ecm_sim* s, int mode) {
-    // a crowd near the limit keeps the form it has: changing it captures the
+static void row_rule(ecm_sim* s, int mode) {
+    // a crowd near a limit keeps the form it has: changing it captures the
     // step graphs anew
-    const int limit = s->row_step ? kRowAgents + kRowAgents / 4 : kRowAgents;
-    s->row_step = mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2 && s->num_agents <= limit;
+    auto small = [&](bool now, int limit) { return s->num_agents <= (now ? limit + limit / 4 : limit); };
+    const bool shape = mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2;
+    s->row_step = shape && small(s->row_step, kRowAgents);
+    s->row_attr = shape && small(s->row_attr, kRowAttrAgents);
 }
 
 static int step_mode(const ecm_sim* s) { return s->log_mlp ? 1 : (s->mlp ? 2 : 0); }
@@ -1572,20 +1578,16 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
     if (half == 0) {
         if (s->timing) HIPCHK(hipEventRecord(s->ev[0], s->stream));
         // block 0 of the count pass also folds the previous step's counters
-        // into the totals and clears them for this step
-        HIPCHK(launch_grid_build(d, s->bsum.p, s->stream));
-        if (s->timing) HIPCHK(hipEventRecord(s->ev[1], s->stream));
-        if (s->row_step) {
-            HIPCHK(launch_row_step(d, s->maxo, s->n_cu, s->stream, s->timing ? s->ev[6] : nullptr));
-            return 0;
-        }
-        // the plain step's main ORCA pass may run inside this kernel (k 5
-        // and 10): its events are published once both are done
-        HIPCHK(launch_attr_knn(d, s->tune.knn_block, mode, s->tune.orca_obst_slots, s->stream,
-                               s->timing ? s->ev[6] : nullptr));
-        // replan and destroy events are final once this kernel is done; its
-        // last block writes them to host memory, and the host handles them
-        // while the ORCA kernels (or, fused, the queue passes) run
+        // into the totals and clears them for this step.  Replan and destroy
+        // events are final once the attraction pass is done: its last block
+        // writes them to host memory, and the host handles them while the
+        // neighbour search and the ORCA kernels run.
+        HIPCHK(launch_grid_attr(d, s->row_attr, s->n_cu, s->stream, s->timing ? s->ev[1] : nullptr));
+        if (s->timing) HIPCHK(hipEventRecord(s->ev[6], s->stream));
+        // the plain step's main ORCA pass may run inside the k-nearest
+        // kernel, or the whole rest of the step in one kernel
+        if (s->row_step) HIPCHK(launch_row_step(d, s->maxo, s->n_cu, s->stream));
+        else HIPCHK(launch_knn(d, s->tune.knn_block, mode, s->tune.orca_obst_slots, s->stream));
         return 0;
     }
     if (s->timing) HIPCHK(hipEventRecord(s->ev[2], s->stream));
@@ -1653,7 +1655,7 @@ static int ensure_step_graph(ecm_sim* s, const DevState& d, int mode) {
     key.frags = mode == 2 ? (const void*)s->mlp->frags.p : nullptr;
     key.pbias = mode == 2 ? (const void*)s->mlp->pbias.p : nullptr;
     key.n_cu = mode == 2 ? s->mlp->n_cu : 0;
-    key.row = s->row_step ? 1 : 0;
+    key.row = (s->row_step ? 1 : 0) | (s->row_attr ? 2 : 0);
     ecm_sim::StepGraph& g = s->graphs[s->cur][d.sorted_in];
     if (g.valid && std::memcmp(&g.key, &key, sizeof(key)) == 0) return 0;
     if (int rc = settle(s)) return rc;      // an earlier launch of g may still run
@@ -1692,7 +1694,7 @@ static int step_once(ecm_sim* s) {
     int rc = prepare_step(s, &d);
     if (rc) return rc;
     const int mode = step_mode(s);
-    row_step_rule(s, mode);
+    row_rule(s, mode);
     bool graph = false;
     if (s->use_graph && !s->timing) {
         rc = ensure_step_graph(s, d, mode);

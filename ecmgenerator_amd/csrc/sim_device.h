@@ -7,6 +7,9 @@
 
 namespace ecm {
 
+// Cell counts that one block of the grid build's prefix sum covers.
+constexpr uint32_t kScanCells = 4096;
+
 // Uniform grid over the world box.  Cell (cx, cy) of a point is
 // floor((p - origin) / cell), clamped to [0, side); NaN maps to 0.
 struct GridDesc {
@@ -104,7 +107,9 @@ struct DevState {
     uint32_t n_keys;        // cells of all environments
     uint32_t* key;          // [n_slots] cell key or 0xffffffff
     uint32_t* rank;         // [n_slots] arrival order of the agent in its cell
-    uint32_t* cell_count;   // [n_keys]   zero between steps (the scan clears it)
+    uint32_t* cell_count;   // [n_keys, padded to scan blocks] zero between steps (the scan clears it)
+    uint32_t* cell_local;   // [n_keys, padded as cell_count] exclusive scan within a scan block
+    uint32_t* bsum;         // [scan blocks] agents per scan block
     uint32_t* cell_start;   // [n_keys + 1] exclusive scan; [n_keys] = active count
     float4* sorted_pr;      // [n_slots] (x, y, radius, id bits)
     float4* sorted_v;       // [n_slots] (vx, vy, preferred speed, environment bits)
@@ -118,7 +123,7 @@ struct DevState {
     int* prev_of;             // [n_slots] this step's sorted position -> previous, -1: none
     int* pos_of;              // [n_slots] agent id -> its sorted position in the last step (k_unsort)
     const int* new_ids;       // agents spawned since the last step, appended to a sorted-entry build
-                              // (their count in acc[15], cleared by k_attr)
+                              // (their count in acc[15], cleared by the last attraction block)
 
     // ---- events ----
     // One list per step, read back by the host after the neighbour pass:

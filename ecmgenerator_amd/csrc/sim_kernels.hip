@@ -179,27 +179,41 @@ __device__ __forceinline__ uint32_t block_excl_scan256(uint32_t v, uint32_t& tot
     __syncthreads();
     return off + inc - v;
 }
-// 1024 counts per block -> local exclusive offsets + block sums; the
-// counts are cleared for the next step
-__global__ __launch_bounds__(256) void k_scan_local(uint32_t* cnt, uint32_t* start, uint32_t* bsum, uint32_t n) {
-    uint32_t base = blockIdx.x * 1024u + threadIdx.x * 4u;
-    uint32_t a[4];
+// The prefix sum of the cell counts takes one launch and part of the scatter:
+// k_scan_local scans kScanCells counts per block into cell_local and the
+// block's total into bsum; every block of the scatter scans the totals again
+// in LDS (a few hundred: under a microsecond, behind its own loads), adds
+// them where it needs a cell's start and writes its share of cell_start.  As
+// a scan of the totals and an add pass of their own these were two launches
+// more, 4-5 us and a 1.5 us gap each whatever the crowd's size.
+static constexpr uint32_t kTopMax = 2048;        // block totals a scatter block scans in LDS
+// kScanCells counts per block; the counts are cleared for the next step.
+// Both arrays are padded to whole blocks.
+__global__ __launch_bounds__(256) void k_scan_local(uint4* cnt, uint4* local, uint32_t* bsum) {
+    uint4* c = cnt + (size_t)blockIdx.x * (kScanCells / 4) + threadIdx.x * 4;
+    uint4 a[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = (base + q < n) ? cnt[base + q] : 0u;
+    for (int q = 0; q < 4; ++q) a[q] = c[q];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        if (base + q < n) cnt[base + q] = 0u;
-    uint32_t loc = a[0] + a[1] + a[2] + a[3];
+    for (int q = 0; q < 4; ++q) c[q] = make_uint4(0, 0, 0, 0);
+    uint32_t sum = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum += a[q].x + a[q].y + a[q].z + a[q].w;
     uint32_t tot;
-    uint32_t ex = block_excl_scan256(loc, tot);
+    uint32_t ex = block_excl_scan256(sum, tot);
+    uint4* o = local + (size_t)blockIdx.x * (kScanCells / 4) + threadIdx.x * 4;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        if (base + q < n) start[base + q] = ex;
-        ex += a[q];
+        uint4 v;
+        v.x = ex; ex += a[q].x;
+        v.y = ex; ex += a[q].y;
+        v.z = ex; ex += a[q].z;
+        v.w = ex; ex += a[q].w;
+        o[q] = v;
     }
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
-// single block: exclusive scan of the block sums, grand total to start[n]
+// More than kTopMax totals: their exclusive scan, by one block.
 __global__ __launch_bounds__(256) void k_scan_top(uint32_t* bsum, uint32_t nb, uint32_t* start, uint32_t n,
                                                   unsigned long long* n_active) {
     uint32_t carry = 0;
@@ -220,9 +234,35 @@ __global__ __launch_bounds__(256) void k_scan_top(uint32_t* bsum, uint32_t nb, u
     }
     if (threadIdx.x == 0) { start[n] = carry; *n_active = carry; }
 }
-__global__ __launch_bounds__(256) void k_scan_add(uint32_t* start, const uint32_t* bsum, uint32_t n) {
-    uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i < n) start[i] += bsum[i >> 10];
+// The block totals as a scatter block sees them: scanned into its LDS, or
+// already scanned in place (nb > kTopMax, by k_scan_top).
+struct Starts {
+    const uint32_t* local;
+    const uint32_t* pre;
+    __device__ __forceinline__ uint32_t at(uint32_t m) const { return local[m] + pre[m / kScanCells]; }
+};
+// The first part of every scatter kernel (256 threads, all of them).
+__device__ __forceinline__ Starts scatter_starts(const DevState& s, uint32_t* top) {
+    const uint32_t nb = (s.n_keys + kScanCells - 1) / kScanCells;
+    Starts S{s.cell_local, s.bsum};
+    if (nb <= kTopMax) {
+        uint32_t carry = 0;
+        for (uint32_t c = 0; c < nb; c += 256u) {
+            const uint32_t i = c + threadIdx.x;
+            uint32_t tot;
+            const uint32_t ex = block_excl_scan256(i < nb ? s.bsum[i] : 0u, tot);
+            if (i < nb) top[i] = carry + ex;
+            carry += tot;
+        }
+        __syncthreads();
+        S.pre = top;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            s.cell_start[s.n_keys] = carry;
+            s.acc[13] = carry;
+        }
+    }
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < s.n_keys; i += gridDim.x * 256u) s.cell_start[i] = S.at(i);
+    return S;
 }
 
 // Counting-sort scatter from the slot-indexed arrays: the sorted position
@@ -232,12 +272,14 @@ __global__ __launch_bounds__(256) void k_scan_add(uint32_t* start, const uint32_
 // there) keeps its neighbour seeds: prev_of and fwd link u and its new
 // position.  Any k distinct agents bound the k-th distance, so seeds stay
 // safe after spawns, removals, writes and loads.
-__global__ void k_grid_scatter(DevState s) {
+__global__ __launch_bounds__(256) void k_grid_scatter(DevState s) {
+    __shared__ uint32_t top[kTopMax];
+    const Starts S = scatter_starts(s, top);
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= s.n_slots) return;
     uint32_t m = s.key[i];
     if (m == kInvalidKey) return;
-    uint32_t slot = s.cell_start[m] + s.rank[i];
+    uint32_t slot = S.at(m) + s.rank[i];
     const float2 p = s.pos_in[i], v = s.vel_in[i];
     s.sorted_pr[slot] = make_float4(p.x, p.y, s.radius[i], __int_as_float(i));
     s.sorted_v[slot] = make_float4(v.x, v.y, s.pref_speed[i], __int_as_float(slot_env(s, i)));
@@ -247,37 +289,6 @@ __global__ void k_grid_scatter(DevState s) {
     const bool was = u >= 0 && u < (int)(uint32_t)s.acc[14] && __float_as_int(s.sorted_pr_old[u].w) == i;
     s.prev_of[slot] = was ? u : -1;
     if (was) s.fwd[u] = (int)slot;
-}
-
-// Counting-sort scatter from the last step's sorted outputs: reads and
-// writes both follow the Morton order, which barely changes from step to
-// step.  Also records the maps between the two orders for the neighbour
-// seeds.
-__global__ void k_grid_scatter_sorted(DevState s) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int n_old = (int)(uint32_t)s.acc[14];
-    if (t >= n_old + (int)(uint32_t)s.acc[15]) return;
-    const uint32_t m = s.key[t];
-    if (m == kInvalidKey) return;
-    const uint32_t slot = s.cell_start[m] + s.rank[t];
-    if (t >= n_old) {                                  // spawned since the last step: no seeds
-        const int id = s.new_ids[t - n_old];
-        const float2 p = s.pos_in[id], v = s.vel_in[id];
-        s.sorted_pr[slot] = make_float4(p.x, p.y, s.radius[id], __int_as_float(id));
-        s.sorted_v[slot] = make_float4(v.x, v.y, s.pref_speed[id], __int_as_float(slot_env(s, id)));
-        s.attr_s[slot] = s.attraction[id];
-        s.path_s[slot] = make_int2(s.path_off[id], s.path_cnt[id]);
-        s.prev_of[slot] = -1;
-        return;
-    }
-    const float2 p = s.pos_s_old[t], v = s.vel_s_old[t];
-    const float4 pr = s.sorted_pr_old[t], sv = s.sorted_v_old[t];
-    s.sorted_pr[slot] = make_float4(p.x, p.y, pr.z, pr.w);
-    s.sorted_v[slot] = make_float4(v.x, v.y, sv.z, sv.w);
-    s.attr_s[slot] = s.attr_s_old[t];
-    s.path_s[slot] = s.path_s_old[t];
-    s.fwd[t] = (int)slot;
-    s.prev_of[slot] = t;
 }
 
 // Agents the host removed since the last step leave a sorted-entry build:
@@ -782,18 +793,29 @@ static constexpr int kKnnBuf = 16;
 static constexpr float kKnnWalkCells = 6.0f;
 static constexpr int kKnnRanges = 4;
 
+// A sorted agent as the attraction pass takes it.
+struct AttrIn {
+    float4 pr, sv;       // sorted_pr, sorted_v
+    int2 pc;             // path_s
+    float2 a0;           // attr_s
+    int prev;            // prev_of
+};
+__device__ __forceinline__ AttrIn attr_in(const DevState& s, int t) {
+    return AttrIn{s.sorted_pr[t], s.sorted_v[t], s.path_s[t], s.attr_s[t], s.prev_of[t]};
+}
+
 // DestroyAgent for sorted agent t: the slot keeps the state it is destroyed
 // with: step-start position and velocity, this step's attraction point, the
 // previous step's preferred and ORCA velocities (already there after a step
 // that started from the slot arrays).  Appends the event and fences it.
-__device__ __forceinline__ void retire_agent(const DevState& s, int t, int id, V2 pos, float4 sv, V2 attr) {
-    s.pos_in[id] = make_float2(pos.x, pos.y);
-    s.vel_in[id] = make_float2(sv.x, sv.y);
+__device__ __forceinline__ void retire_agent(const DevState& s, const AttrIn& in, V2 attr) {
+    const int id = __float_as_int(in.pr.w);
+    s.pos_in[id] = make_float2(in.pr.x, in.pr.y);
+    s.vel_in[id] = make_float2(in.sv.x, in.sv.y);
     s.attraction[id] = make_float2(attr.x, attr.y);
-    const int qp = s.prev_of[t];
-    if (s.sorted_in && qp >= 0) {
-        s.pref_vel[id] = s.pref_vel_s_old[qp];
-        if (s.v_orca) s.v_orca[id] = s.v_orca_s_old[qp];
+    if (s.sorted_in && in.prev >= 0) {
+        s.pref_vel[id] = s.pref_vel_s_old[in.prev];
+        if (s.v_orca) s.v_orca[id] = s.v_orca_s_old[in.prev];
     }
     s.active[id] = 0;
     const uint32_t q = atomicAdd(s.events_n, 1u);
@@ -801,28 +823,20 @@ __device__ __forceinline__ void retire_agent(const DevState& s, int t, int id, V
     __threadfence();
 }
 
-// One sorted agent's goal check, attraction point and steering (with the
-// destroy or replan request they may make).  Returns whether it appended an
-// event, after fencing it device-wide.
-__device__ __forceinline__ bool attr_agent(const DevState& s) {
-    const uint32_t n_active = s.cell_start[s.n_keys];
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= (int)n_active) return false;
-    const float4 pr = s.sorted_pr[t];
-    const float4 sv = s.sorted_v[t];
-    const int2 pc = s.path_s[t];
-    const int id = __float_as_int(pr.w);
-    const V2 pos = mk(pr.x, pr.y);
-    const EnvDesc& E = env_of_sorted(s, sv);
+// The goal check, attraction point and steering of the agent at sorted
+// position t (with the destroy or replan request it may make).  Returns
+// whether it appended an event, after fencing it device-wide.
+__device__ __forceinline__ bool attr_agent(const DevState& s, int t, const AttrIn& in) {
+    const V2 pos = mk(in.pr.x, in.pr.y);
+    const EnvDesc& E = env_of_sorted(s, in.sv);
 
     // UpdateAttractionPointSystem (Simulator.cpp:538-590)
-    const int np = pc.y;
-    const float2* path = s.path_pts + pc.x;
+    const int np = in.pc.y;
+    const float2* path = s.path_pts + in.pc.x;
     float2 gg = path[np - 1];
     float gx = pos.x - gg.x, gy = pos.y - gg.y;
     float dGoal = gx * gx + gy * gy;
-    float2 a0 = s.attr_s[t];
-    V2 attr = mk(a0.x, a0.y);
+    V2 attr = mk(in.a0.x, in.a0.y);
     bool alive = true, event = false;
     uint32_t fb = 0;
     if (dGoal < s.arrival_r2) {
@@ -834,7 +848,7 @@ __device__ __forceinline__ bool attr_agent(const DevState& s) {
         else {
             // UpdatePath(e, currentPosition, goal) with the step-start position
             uint32_t q = atomicAdd(s.events_n, 1u);
-            s.events[q] = make_int4(id, __float_as_int(pos.x), __float_as_int(pos.y), t);
+            s.events[q] = make_int4(__float_as_int(in.pr.w), __float_as_int(pos.x), __float_as_int(pos.y), t);
             event = true;
         }
     }
@@ -842,11 +856,11 @@ __device__ __forceinline__ bool attr_agent(const DevState& s) {
     if (fb) atomicAdd(&s.stats[2], 1u);
     s.dead_s[t] = alive ? 0 : 1;
     if (!alive) {
-        retire_agent(s, t, id, pos, sv, attr);
+        retire_agent(s, in, attr);
         return true;
     }
     // ApplySteeringForce (Simulator.cpp:638-657)
-    const float speed = sv.z;
+    const float speed = in.sv.z;
     V2 des = normalize(attr - pos) * speed;
     s.pref_vel_s[t] = make_float2(des.x, des.y);
     if (event) __threadfence();
@@ -907,18 +921,74 @@ __device__ __forceinline__ void publish_if_last(const DevState& s) {
     __syncthreads();
     if (threadIdx.x == 0) {
         *s.blocks_done = 0u;
+        s.acc[15] = 0;                       // every block's grid build has used it
         __threadfence_system();
         *(volatile uint32_t*)s.host_xfer = (uint32_t)s.acc[12];
     }
 }
 
-// Goal checks, attraction points and steering of every agent; the block
-// that finishes last publishes the step's events, so the host plans the
-// replans while the neighbour search and the ORCA passes run.  No LDS: the
-// IRM's dependent loads are hidden by as many waves as the registers allow.
+// Goal checks, attraction points and steering of every agent, after a grid
+// build from the slot arrays (whose order no wavefront's loads would share);
+// the block that finishes last publishes the step's events, so the host plans
+// the replans while the neighbour search and the ORCA passes run.  The IRM's
+// dependent loads are hidden by as many waves as the registers allow.
 __global__ __launch_bounds__(256) void k_attr(DevState s) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) s.acc[15] = 0;   // the grid build has used it
-    attr_agent(s);
+    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    if (t < (int)s.cell_start[s.n_keys]) attr_agent(s, t, attr_in(s, t));
+    publish_if_last(s);
+}
+
+// An element of a build from the last step's sorted outputs: agent t of the
+// last step, or the (t - n_old)-th agent spawned since.  Stores its state at
+// its sorted position `slot` with the maps between the two orders for the
+// neighbour seeds, and returns it.
+__device__ __forceinline__ AttrIn scatter_agent(const DevState& s, int t, int n_old, int slot, bool write) {
+    AttrIn in;
+    if (t >= n_old) {                                  // spawned since the last step: no seeds
+        const int id = s.new_ids[t - n_old];
+        const float2 p = s.pos_in[id], v = s.vel_in[id];
+        in.pr = make_float4(p.x, p.y, s.radius[id], __int_as_float(id));
+        in.sv = make_float4(v.x, v.y, s.pref_speed[id], __int_as_float(slot_env(s, id)));
+        in.a0 = s.attraction[id];
+        in.pc = make_int2(s.path_off[id], s.path_cnt[id]);
+        in.prev = -1;
+    } else {
+        const float2 p = s.pos_s_old[t], v = s.vel_s_old[t];
+        const float4 pr = s.sorted_pr_old[t], sv = s.sorted_v_old[t];
+        in.pr = make_float4(p.x, p.y, pr.z, pr.w);
+        in.sv = make_float4(v.x, v.y, sv.z, sv.w);
+        in.a0 = s.attr_s_old[t];
+        in.pc = s.path_s_old[t];
+        in.prev = t;
+        if (write) s.fwd[t] = slot;
+    }
+    if (write) {
+        s.sorted_pr[slot] = in.pr;
+        s.sorted_v[slot] = in.sv;
+        s.path_s[slot] = in.pc;
+        s.prev_of[slot] = in.prev;
+    }
+    return in;
+}
+
+// Counting-sort scatter from the last step's sorted outputs, and the
+// attraction pass on what it holds in registers: reads and writes both
+// follow the Morton order, which barely changes from step to step.  One
+// kernel instead of two: the attraction pass does not read back 52 B per
+// agent, and the scatter's stores go out behind its dependent loads.  The
+// last block publishes the events, as in k_attr.
+__global__ __launch_bounds__(256) void k_scatter_attr(DevState s) {
+    __shared__ uint32_t top[kTopMax];
+    const Starts S = scatter_starts(s, top);
+    const int t = xcd_block() * blockDim.x + threadIdx.x;
+    const int n_old = (int)(uint32_t)s.acc[14];
+    if (t < n_old + (int)(uint32_t)s.acc[15]) {
+        const uint32_t m = s.key[t];
+        if (m != kInvalidKey) {
+            const int slot = (int)(S.at(m) + s.rank[t]);
+            attr_agent(s, slot, scatter_agent(s, t, n_old, slot, true));
+        }
+    }
     publish_if_last(s);
 }
 
@@ -2015,18 +2085,28 @@ static inline int round8(int n) { return (n + 7) & ~7; }
 // From the last step's sorted outputs (s.sorted_in) the count and scatter
 // passes cover its agents (the count is read on the device); from the slot
 // arrays, every slot.  The launch shapes depend only on the capacity, so
-// one captured graph serves each entry for any agent count.
-hipError_t launch_grid_build(const DevState& s, uint32_t* bsum, hipStream_t st) {
-    const uint32_t G = s.n_keys;
-    const dim3 ga(cdiv(s.n_slots, 256)), b(256);
+// one captured graph serves each entry for any agent count.  The attraction
+// pass is part of the scatter, or (from the slot arrays) follows it; `row`:
+// with 16 lanes per agent.  `mid`, when not null, is recorded before them.
+hipError_t launch_grid_attr(const DevState& s, bool row, int n_cu, hipStream_t st, hipEvent_t mid) {
+    const dim3 ga(round8(cdiv(s.n_slots, 256))), b(256);
+    // 16 agents per block, strided: no more blocks than stay resident
+    const dim3 gr(std::min(round8(cdiv(s.n_slots, 16)), round8(std::max(1, n_cu) * 8)));
     if (s.sorted_in) hipLaunchKernelGGL(k_grid_count_sorted, ga, b, 0, st, s);
     else hipLaunchKernelGGL(k_grid_count, ga, b, 0, st, s);
-    const uint32_t nb = (G + 1023u) / 1024u;
-    hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(256), 0, st, s.cell_count, s.cell_start, bsum, G);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, st, bsum, nb, s.cell_start, G, s.acc + 13);
-    hipLaunchKernelGGL(k_scan_add, dim3(cdiv(G, 256)), dim3(256), 0, st, s.cell_start, (const uint32_t*)bsum, G);
-    if (s.sorted_in) hipLaunchKernelGGL(k_grid_scatter_sorted, ga, b, 0, st, s);
-    else hipLaunchKernelGGL(k_grid_scatter, ga, b, 0, st, s);
+    const uint32_t nb = (s.n_keys + kScanCells - 1) / kScanCells;
+    hipLaunchKernelGGL(k_scan_local, dim3(nb), b, 0, st, (uint4*)s.cell_count, (uint4*)s.cell_local, s.bsum);
+    if (nb > kTopMax) hipLaunchKernelGGL(k_scan_top, dim3(1), b, 0, st, s.bsum, nb, s.cell_start, s.n_keys, s.acc + 13);
+    if (mid && s.sorted_in) (void)hipEventRecord(mid, st);
+    if (s.sorted_in) {
+        if (row) hipLaunchKernelGGL(k_scatter_attr_row, gr, b, 0, st, s);
+        else hipLaunchKernelGGL(k_scatter_attr, ga, b, 0, st, s);
+    } else {
+        hipLaunchKernelGGL(k_grid_scatter, ga, b, 0, st, s);
+        if (mid) (void)hipEventRecord(mid, st);
+        if (row) hipLaunchKernelGGL(k_attr_row, gr, b, 0, st, s);
+        else hipLaunchKernelGGL(k_attr, ga, b, 0, st, s);
+    }
     return hipGetLastError();
 }
 
@@ -2118,25 +2198,17 @@ static void launch_orca_k(const DevState& s, int maxo, int mode, int oslots, int
     }
 }
 
-// The passes with 16 lanes per agent (row_kernels.h): the whole rest of the
-// plain step after the grid build.  Grids of at most 32 wavefronts per CU,
-// strided, so that spare slots of a large pool cost nothing.
-hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st, hipEvent_t mid) {
-    const int cap = std::max(1, n_cu) * 32;
-    const dim3 ga(std::min(round8(cdiv(s.n_slots, 16)), round8(cap / 4)));
-    hipLaunchKernelGGL(k_attr_row, ga, dim3(256), 0, st, s);
-    if (mid) (void)hipEventRecord(mid, st);
+// The neighbour search and ORCA with 16 lanes per agent (row_kernels.h): the
+// rest of the plain step.  A grid of at most 32 wavefronts per CU, strided,
+// so that spare slots of a large pool cost nothing.
+hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st) {
     const int row_f4 = std::max(maxo, kRowLdsBytes / 16);
-    hipLaunchKernelGGL(k_row_step, dim3(std::min(round8(cdiv(s.n_slots, 4)), round8(cap))), dim3(64),
+    hipLaunchKernelGGL(k_row_step, dim3(std::min(round8(cdiv(s.n_slots, 4)), round8(std::max(1, n_cu) * 32))), dim3(64),
                        (size_t)row_f4 * 4 * sizeof(float4), st, s, maxo, row_f4);
     return hipGetLastError();
 }
 
-// `mid`, when not null, is recorded between the attraction pass and the
-// k-nearest pass.
-hipError_t launch_attr_knn(const DevState& s, int block, int mode, int oslots, hipStream_t st, hipEvent_t mid) {
-    hipLaunchKernelGGL(k_attr, dim3(round8(cdiv(s.n_slots, 256))), dim3(256), 0, st, s);
-    if (mid) (void)hipEventRecord(mid, st);
+hipError_t launch_knn(const DevState& s, int block, int mode, int oslots, hipStream_t st) {
     if (block == 16 && orca_fused(s.k, mode, oslots)) {
         // 16 agents per wavefront of 64 threads
         const dim3 gs(round8(cdiv(s.n_slots, 16))), bs(64);
