@@ -277,6 +277,7 @@ struct ecm_sim {
         hipGraphExec_t exec[2] = {nullptr, nullptr};
     };
     bool use_graph = false;
+    bool idle = true;                           // nothing queued on the stream since it was last waited for
     bool row_step = false, row_attr = false;    // 16 lanes per agent (row_rule)
     StepGraph graphs[2][2];                     // [parity][entry from the sorted outputs]
     std::string graph_error;
@@ -375,6 +376,7 @@ static float bits_to_float(int v) {
 // every entry point that reads or replaces device data settles first.
 static int settle(ecm_sim* s) {
     HIPCHK(hipStreamSynchronize(s->stream));
+    s->idle = true;
     return 0;
 }
 // settle + bring the slot-indexed agent arrays up to date (defined after
@@ -1695,8 +1697,15 @@ static int step_once(ecm_sim* s) {
     if (rc) return rc;
     const int mode = step_mode(s);
     row_rule(s, mode);
+    // A step replays its graph when it finds the stream idle: one call then
+    // puts all its kernels behind each other.  Behind a step that still runs
+    // (a loop of steps with nothing read in between) its kernels are
+    // launched one by one: that is hidden by the running step, and a graph's
+    // start leaves the GPU idle for 7-13 us (20 steps of 5,000 agents 1143 ->
+    // 1025 us, of 100,000 3434 -> 3285; 500 agents read after every step 1304
+    // -> 1256 with the graph).
     bool graph = false;
-    if (s->use_graph && !s->timing) {
+    if (s->use_graph && !s->timing && s->idle) {
         rc = ensure_step_graph(s, d, mode);
         if (rc < 0) return rc;
         if (rc == 0) graph = true;
@@ -1706,6 +1715,7 @@ static int step_once(ecm_sim* s) {
     if (graph) HIPCHK(hipGraphLaunch(s->graphs[s->cur][d.sorted_in].exec[0], s->stream));
     else if ((rc = enqueue_device_half(s, d, mode, 0)) != 0 || (rc = enqueue_device_half(s, d, mode, 1)) != 0)
         return rc;
+    s->idle = false;
     const uint32_t peek = (uint32_t)std::min(ecm_sim::kEventPeek, s->prm.max_agents);
     if ((rc = wait_published(s, ++s->step_seq)) != 0) return rc;
     const uint32_t ne = s->h_xfer[1];
@@ -1908,8 +1918,7 @@ extern "C" int ecm_sim_autotune(ecm_sim* s, int steps, ecm_sim_tuning* out) {
 
 extern "C" int ecm_sim_sync(ecm_sim* s) {
     if (!s) return fail(ECM_E_ARG, "null handle");
-    HIPCHK(hipStreamSynchronize(s->stream));
-    return 0;
+    return settle(s);
 }
 
 static int component_buf(ecm_sim* s, int c, void** p, size_t* elem) {
@@ -1947,8 +1956,7 @@ extern "C" int ecm_sim_read(ecm_sim* s, int c, void* dst, size_t bytes) {
         return rc_;
     }
     HIPCHK(hipMemcpyAsync(dst, p, bytes, hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
-    return 0;
+    return settle(s);
 }
 
 extern "C" int ecm_sim_write(ecm_sim* s, int c, const void* src, size_t bytes) {
@@ -1962,7 +1970,7 @@ extern "C" int ecm_sim_write(ecm_sim* s, int c, const void* src, size_t bytes) {
     (void)hipSetDevice(s->dev);
     if (int rc_ = sync_state(s)) return rc_;
     HIPCHK(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     const float* f = (const float*)src;
     if (c == ECM_C_CLEARANCE)
         for (size_t i = 0; i < N; ++i) { s->h_radius[i] = f[i]; s->max_radius = std::max(s->max_radius, f[i]); }

@@ -105,7 +105,9 @@ int ecm_sim_set_replan_threads(ecm_sim* s, int n);
  * hipGraph (one per position-buffer parity; the host reads the replan
  * events from host-mapped memory while the graph still runs) and
  * replayed, recaptured whenever buffers, parameters or the launch shape
- * change.  Steps with timing on run eagerly.  If capture fails the handle
+ * change.  Steps with timing on run eagerly, and so does a step that
+ * begins while the one before it still runs, where launching kernel by
+ * kernel is the faster way.  If capture fails the handle
  * falls back to eager launches; ecm_sim_graph_status reports whether
  * graphs are in use and, if not, why. */
 int ecm_sim_set_graph(ecm_sim* s, int on);
