@@ -62,6 +62,17 @@ __host__ __device__ constexpr int hidden_perm(int k) {
     return 32 * ((k / 16) / 2) + 16 * ((k / 16) % 2) + 8 * (((k % 16) % 8) / 4) + 4 * ((k % 16) / 8) + ((k % 16) % 4);
 }
 
+// Training packs the same fragments, their K axes in order, and behind them
+// the transposed weights of layers 4, 3 and 2 for the backward chain: A
+// operands whose rows are the layer's inputs and whose K axis is its outputs.
+constexpr int kFragB4 = kNFrags, kFragB3 = kFragB4 + 4, kFragB2 = kFragB3 + 32, kNTrainFrags = kFragB2 + 32;
+constexpr int kNBiasParams = 3 * kHid + kOut;        // bias gradients: b1, b2, b3, b4
+
+// Weight-gradient jobs of one batch chunk (k_train_dw), each an M x N block
+// of partial sums, row-major as the weights.
+constexpr int kDwOff3 = 0, kDwOff2 = kDwOff3 + kHid * kHid, kDwOff1 = kDwOff2 + kHid * kHid,
+              kDwOff4 = kDwOff1 + kHid * kInPad, kDwFloats = kDwOff4 + kOut * kHid;
+
 // Label word of a logged sample: bits 0..13 active slots, 16..29 slots
 // that exist (a constraint is behind the slot), bit 30 every active
 // constraint is behind some slot.

@@ -1,6 +1,6 @@
 // mlp_api.cpp -- host runtime behind include/ecm_mlp.h: parameters,
 // dataset, the training loop (forward, backward and Adam on the GPU with
-// the kernels of mlp_kernels.hip) and host-data entry points for checks.
+// the kernels of mlp_kernels.hip) and host-data entry points.
 #include "mlp_host.h"
 
 #include <algorithm>
@@ -16,9 +16,8 @@ using namespace ecm::mlp;
 static uint16_t f32_to_bf16_rne(float f) {
     uint32_t u;
     std::memcpy(&u, &f, 4);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0;          // NaN
-    const uint32_t r = ((u >> 16) & 1u) + 0x7fffu;
-    return (uint16_t)((u + r) >> 16);
+    const uint32_t r = (u + (((u >> 16) & 1u) + 0x7fffu)) >> 16;
+    return (uint16_t)((u & 0x7fffffffu) > 0x7f800000u ? 0x7fc0u : r);          // NaN: quiet
 }
 static float bf16_to_f32(uint16_t h) {
     uint32_t u = (uint32_t)h << 16;
@@ -40,10 +39,10 @@ extern "C" int ecm_mlp_create(uint64_t seed, ecm_mlp** out) {
     int rc = 0;
     if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) rc = fail(ECM_E_HIP, "stream create failed");
     if (!rc) rc = m->params.alloc(kNParams);
-    if (!rc) rc = m->grads.alloc(kNParams);
+    if (!rc) rc = m->grads.alloc(kNParams + 1);
     if (!rc) rc = m->adam_m.alloc(kNParams);
     if (!rc) rc = m->adam_v.alloc(kNParams);
-    if (!rc) rc = m->wbf.alloc(kNParams);
+    if (!rc) rc = m->tfrags.alloc((size_t)kNTrainFrags * 64);
     if (!rc) rc = m->frags.alloc((size_t)kNFrags * 64);
     if (!rc) rc = m->pbias.alloc(kNBias);
     if (!rc) rc = m->ds_count.alloc(1);
@@ -77,11 +76,10 @@ extern "C" int ecm_mlp_destroy(ecm_mlp* m) {
     if (!m) return 0;
     (void)hipSetDevice(m->dev);
     (void)hipDeviceSynchronize();
-    for (auto* b : {&m->params, &m->grads, &m->adam_m, &m->adam_v, &m->pbias, &m->z1, &m->z2, &m->z3, &m->y, &m->dyf,
-                    &m->dh, &m->dzf, &m->loss})
+    for (auto* b : {&m->params, &m->grads, &m->adam_m, &m->adam_v, &m->pbias, &m->y, &m->part, &m->bias_part})
         b->release();
-    for (auto* b : {&m->wbf, &m->h1, &m->h2, &m->h3, &m->dy, &m->dz}) b->release();
-    m->frags.release(); m->ds_x.release(); m->xb.release();
+    for (auto* b : {&m->frags, &m->tfrags, &m->ds_x, &m->xb, &m->h1, &m->h2, &m->h3, &m->dz1, &m->dz2, &m->dz3, &m->dy})
+        b->release();
     m->ds_label.release(); m->ds_count.release(); m->lb.release();
     m->ds_v.release(); m->vb.release(); m->perm.release();
     if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -104,10 +102,10 @@ extern "C" int ecm_mlp_set_params(ecm_mlp* m, const float* in, int n) {
     (void)hipSetDevice(m->dev);
     HIPCHK(hipDeviceSynchronize());          // a simulator step may still read the packed weights
     HIPCHK(hipMemcpyAsync(m->params.p, in, kNParams * sizeof(float), hipMemcpyHostToDevice, m->stream));
-    HIPCHK(launch_to_bf16(m->params.p, m->wbf.p, kNParams, m->stream));
     HIPCHK(launch_fill_f32(m->adam_m.p, 0.0f, kNParams, m->stream));
     HIPCHK(launch_fill_f32(m->adam_v.p, 0.0f, kNParams, m->stream));
     m->adam_t = 0;
+    m->tpacked = false;
     int rc = ecm_mlp_pack(m);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(m->stream));
@@ -188,69 +186,69 @@ extern "C" int ecm_mlp_dataset_read(ecm_mlp* m, int64_t first, int n, float* x, 
 }
 
 // ---------------------------------------------------------------- training
-static int ensure_ws(ecm_mlp* m, int B) {
-    if (m->ws_batch >= B) return 0;
+static int ensure_in(ecm_mlp* m, int B) {
+    if (m->in_batch >= B) return 0;
     int rc = m->xb.alloc((size_t)B * 8);
     if (!rc) rc = m->lb.alloc(B);
     if (!rc) rc = m->vb.alloc(B);
-    for (auto* b : {&m->z1, &m->z2, &m->z3, &m->dh, &m->dzf})
-        if (!rc) rc = b->alloc((size_t)B * kHid);
     if (!rc) rc = m->y.alloc((size_t)B * kOut);
-    if (!rc) rc = m->dyf.alloc((size_t)B * kOut);
-    if (!rc) rc = m->loss.alloc(1);
-    for (auto* b : {&m->h1, &m->h2, &m->h3, &m->dz})
-        if (!rc) rc = b->alloc((size_t)B * kHid);
-    if (!rc) rc = m->dy.alloc((size_t)B * kOut);
+    m->in_batch = rc ? 0 : B;
+    return rc;
+}
+
+static int ensure_ws(ecm_mlp* m, int B) {
+    if (m->ws_batch >= B) return 0;
+    m->ws_batch = 0;
+    int rc = m->dy.alloc((size_t)B * 2);
+    for (auto* b : {&m->h1, &m->h2, &m->h3, &m->dz1, &m->dz2, &m->dz3})
+        if (!rc) rc = b->alloc((size_t)B * 16);
+    if (!rc) rc = m->part.alloc((size_t)train_chunks(B) * kDwFloats);
+    if (!rc) rc = m->bias_part.alloc((size_t)m->n_cu * (kNBiasParams + 1));
     if (rc) return rc;
     m->ws_batch = B;
     return 0;
 }
 
-// Forward and backward of the batch staged in xb / lb / vb; adds the
-// gradient into grads and the batch loss into loss[0].
-static int fwd_bwd(ecm_mlp* m, int B, float pos_w, float vel_w) {
-    hipStream_t st = m->stream;
-    const __bf16* X = reinterpret_cast<const __bf16*>(m->xb.p);
-    const __bf16* W = m->wbf.p;
-    const float* P = m->params.p;
-    float* G = m->grads.p;
-    const int sk = std::max(1, B / 512);
-    // forward: Z = X W^T, H = silu(Z + b)
-    HIPCHK(launch_gemm(B, kHid, kInPad, X, kInPad, 1, W + kOffW1, kInPad, 1, m->z1.p, kHid, 1, 0, 1, st));
-    HIPCHK(launch_bias_silu(m->z1.p, P + kOffB1, m->h1.p, B, kHid, st));
-    HIPCHK(launch_gemm(B, kHid, kHid, m->h1.p, kHid, 1, W + kOffW2, kHid, 1, m->z2.p, kHid, 1, 0, 1, st));
-    HIPCHK(launch_bias_silu(m->z2.p, P + kOffB2, m->h2.p, B, kHid, st));
-    HIPCHK(launch_gemm(B, kHid, kHid, m->h2.p, kHid, 1, W + kOffW3, kHid, 1, m->z3.p, kHid, 1, 0, 1, st));
-    HIPCHK(launch_bias_silu(m->z3.p, P + kOffB3, m->h3.p, B, kHid, st));
-    HIPCHK(launch_gemm(B, kOut, kHid, m->h3.p, kHid, 1, W + kOffW4, kHid, 1, m->y.p, kOut, 1, 0, 1, st));
-    HIPCHK(launch_head(m->y.p, P + kOffB4, m->lb.p, m->vb.p, m->dy.p, m->dyf.p, m->loss.p, B, pos_w, vel_w, st));
-    // layer 4: dW4 += dY^T H3, db4 += sum dY, dH3 = dY W4
-    HIPCHK(launch_gemm(kOut, kHid, B, m->dy.p, 1, kOut, m->h3.p, 1, kHid, G + kOffW4, kHid, 1, 1, sk, st));
-    HIPCHK(launch_colsum(m->dyf.p, B, kOut, G + kOffB4, st));
-    HIPCHK(launch_gemm(B, kHid, kOut, m->dy.p, kOut, 1, W + kOffW4, 1, kHid, m->dh.p, kHid, 1, 0, 1, st));
-    // hidden layers 3, 2, 1
-    const __bf16* Hin[3] = {X, m->h1.p, m->h2.p};
-    const float* Zs[3] = {m->z1.p, m->z2.p, m->z3.p};
-    const int offW[3] = {kOffW1, kOffW2, kOffW3}, offB[3] = {kOffB1, kOffB2, kOffB3};
-    const int nin[3] = {kInPad, kHid, kHid};
-    for (int l = 2; l >= 0; --l) {
-        HIPCHK(launch_silu_bwd(m->dh.p, Zs[l], m->dz.p, m->dzf.p, B, kHid, st));
-        HIPCHK(launch_colsum(m->dzf.p, B, kHid, G + offB[l], st));
-        HIPCHK(launch_gemm(kHid, nin[l], B, m->dz.p, 1, kHid, Hin[l], 1, nin[l], G + offW[l], nin[l], 1, 1, sk, st));
-        if (l > 0)
-            HIPCHK(launch_gemm(B, nin[l], kHid, m->dz.p, kHid, 1, W + offW[l], 1, nin[l], m->dh.p, kHid, 1, 0, 1, st));
-    }
+// The training fragments of the current parameters: packed at the first use
+// after the parameters were set, kept current by the Adam steps.
+static int pack_train(ecm_mlp* m) {
+    if (m->tpacked) return 0;
+    HIPCHK(launch_train_pack(m->params.p, m->tfrags.p, m->stream));
+    m->tpacked = true;
     return 0;
 }
 
+// The workspace and loss settings of a batch of B rows; the rows, the Adam
+// constants and where the gradient goes are the caller's.
+static TrainBatch train_batch(ecm_mlp* m, int B, float pos_w, float vel_w) {
+    TrainBatch t{};
+    t.n = B;
+    t.pos_w = pos_w;
+    t.vel_w = vel_w;
+    t.frags = m->tfrags.p;
+    t.params = m->params.p;
+    t.h[0] = m->h1.p; t.h[1] = m->h2.p; t.h[2] = m->h3.p;
+    t.dz[0] = m->dz1.p; t.dz[1] = m->dz2.p; t.dz[2] = m->dz3.p;
+    t.dy = m->dy.p;
+    t.bias_part = m->bias_part.p;
+    t.max_blocks = m->n_cu;
+    t.part = m->part.p;
+    t.w = m->params.p;
+    t.m = m->adam_m.p;
+    t.v2 = m->adam_v.p;
+    t.loss = m->grads.p + kNParams;
+    return t;
+}
+
 static int stage_host_batch(ecm_mlp* m, const float* x, const uint32_t* label, const float* v, int n) {
-    std::vector<uint16_t> xb((size_t)n * 64);
-    for (size_t i = 0; i < xb.size(); ++i) xb[i] = f32_to_bf16_rne(x[i]);
-    HIPCHK(hipMemcpyAsync(m->xb.p, xb.data(), xb.size() * 2, hipMemcpyHostToDevice, m->stream));
+    const size_t nx = (size_t)n * 64;
+    if (m->h_x.size() < nx) m->h_x.resize(nx);
+    uint16_t* xb = m->h_x.data();
+    for (size_t i = 0; i < nx; ++i) xb[i] = f32_to_bf16_rne(x[i]);
+    HIPCHK(hipMemcpyAsync(m->xb.p, xb, nx * 2, hipMemcpyHostToDevice, m->stream));
     if (label) HIPCHK(hipMemcpyAsync(m->lb.p, label, (size_t)n * 4, hipMemcpyHostToDevice, m->stream));
     if (v) HIPCHK(hipMemcpyAsync(m->vb.p, v, (size_t)n * 8, hipMemcpyHostToDevice, m->stream));
-    HIPCHK(hipStreamSynchronize(m->stream));      // xb (host vector) must outlive the copy
-    return 0;
+    return 0;                                     // every caller waits for the stream before it returns
 }
 
 extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* label, const float* v, int n,
@@ -258,13 +256,18 @@ extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* lab
     if (!m || !x || !label || !v || n < 1 || !loss || !grad) return fail(ECM_E_ARG, "bad arguments");
     (void)hipSetDevice(m->dev);
     int rc = ensure_ws(m, n);
+    if (!rc) rc = ensure_in(m, n);
     if (!rc) rc = stage_host_batch(m, x, label, v, n);
     if (rc) return rc;
-    HIPCHK(launch_fill_f32(m->grads.p, 0.0f, kNParams, m->stream));
-    HIPCHK(launch_fill_f32(m->loss.p, 0.0f, 1, m->stream));
-    rc = fwd_bwd(m, n, pos_weight, vel_weight);
-    if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(loss, m->loss.p, sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    if ((rc = pack_train(m)) != 0) return rc;
+    TrainBatch t = train_batch(m, n, pos_weight, vel_weight);
+    t.first = true;
+    t.x = m->xb.p;
+    t.label = m->lb.p;
+    t.v = m->vb.p;
+    t.grad = m->grads.p;
+    HIPCHK(launch_train_batch(t, m->stream));
+    HIPCHK(hipMemcpyAsync(loss, t.loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipMemcpyAsync(grad, m->grads.p, kNParams * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
     return 0;
@@ -273,7 +276,7 @@ extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* lab
 extern "C" int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y) {
     if (!m || !x || !y || n < 1) return fail(ECM_E_ARG, "bad arguments");
     (void)hipSetDevice(m->dev);
-    int rc = ensure_ws(m, n);
+    int rc = ensure_in(m, n);
     if (!rc) rc = stage_host_batch(m, x, nullptr, nullptr, n);
     if (rc) return rc;
     HIPCHK(launch_mlp_infer(m->xb.p, 0, nullptr, n, m->frags.p, m->pbias.p, 0.0f, m->lb.p, nullptr, m->y.p, m->n_cu,
@@ -284,13 +287,11 @@ extern "C" int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y) {
 }
 
 // ------------------------------------------- forward without allocation
-// Scratch of ecm_mlp_forward_noalloc: the BF16 features ([n][64]) and the
-// proposal masks ([n]) of up to ECM_MLP_NOALLOC_MAX_SAMPLES samples.  Every
-// GPU holds its own copy until the process ends.  Nothing in it has to
-// start at zero: the conversion kernel writes every feature the network
-// reads and the network writes every mask.
-constexpr size_t kNoAllocFeatBytes = (size_t)ECM_MLP_NOALLOC_MAX_SAMPLES * kInPad * 2;
-constexpr size_t kNoAllocBytes = kNoAllocFeatBytes + (size_t)ECM_MLP_NOALLOC_MAX_SAMPLES * 4;
+// Scratch of ecm_mlp_forward_noalloc: the proposal masks ([n]) of up to
+// ECM_MLP_NOALLOC_MAX_SAMPLES samples.  Every GPU holds its own copy until
+// the process ends.  Nothing in it has to start at zero: the network writes
+// every mask.
+constexpr size_t kNoAllocBytes = (size_t)ECM_MLP_NOALLOC_MAX_SAMPLES * 4;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
 // Device address of `scratch` on device `dev`, looked up once per device
@@ -320,10 +321,10 @@ extern "C" int ecm_mlp_forward_noalloc(ecm_mlp* m, const float* x, int n, float*
     unsigned char* base = nullptr;
     int rc = scratch_address(m->dev, &base);
     if (rc) return rc;
-    uint16_t* xb = reinterpret_cast<uint16_t*>(base);
-    uint32_t* mask = reinterpret_cast<uint32_t*>(base + kNoAllocFeatBytes);
-    HIPCHK(launch_f32_to_bf16_rne(x, xb, (long)n * kInPad, m->stream));
-    HIPCHK(launch_mlp_infer(xb, 0, nullptr, n, m->frags.p, m->pbias.p, 0.0f, mask, nullptr, y, m->n_cu, m->stream));
+    // the network reads the FP32 rows itself, rounding as the host staging of
+    // ecm_mlp_forward does
+    HIPCHK(launch_mlp_infer(x, 2, nullptr, n, m->frags.p, m->pbias.p, 0.0f, reinterpret_cast<uint32_t*>(base), nullptr,
+                            y, m->n_cu, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
     return 0;
 }
@@ -340,32 +341,46 @@ extern "C" int ecm_mlp_train(ecm_mlp* m, int epochs, int batch, float lr, float 
     rc = ensure_ws(m, batch);
     if (!rc && m->perm.n < (size_t)n) rc = m->perm.alloc((size_t)n);
     if (rc) return rc;
-    std::vector<int64_t> perm((size_t)n);
-    for (int64_t i = 0; i < n; ++i) perm[i] = i;
+    // Fisher-Yates with the seeded generator (reproducible across hosts); the
+    // next epoch's order is drawn while the GPU works on this one's
+    std::vector<int32_t> order[2];      // (the capacity fits an int)
     std::mt19937_64 rng(seed);
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const int64_t nb = n / batch;
-    for (int e = 0; e < epochs; ++e) {
-        // Fisher-Yates with the seeded generator (reproducible across hosts)
+    auto shuffle = [&](std::vector<int32_t>& p) {
         for (int64_t i = n - 1; i > 0; --i) {
             const int64_t j = (int64_t)(rng() % (uint64_t)(i + 1));
-            std::swap(perm[i], perm[j]);
+            std::swap(p[i], p[j]);
         }
-        HIPCHK(hipMemcpyAsync(m->perm.p, perm.data(), (size_t)n * sizeof(int64_t), hipMemcpyHostToDevice, m->stream));
-        HIPCHK(launch_fill_f32(m->loss.p, 0.0f, 1, m->stream));
+    };
+    order[0].resize((size_t)n);
+    for (int64_t i = 0; i < n; ++i) order[0][i] = (int32_t)i;
+    if (epochs > 0) shuffle(order[0]);
+    const int64_t nb = n / batch;
+    TrainBatch t = train_batch(m, batch, pos_weight, vel_weight);
+    t.x = m->ds_x.p;
+    t.label = m->ds_label.p;
+    t.v = m->ds_v.p;
+    t.lr = lr;
+    t.b1 = 0.9f;
+    t.b2 = 0.999f;
+    t.eps = 1e-8f;
+    if ((rc = pack_train(m)) != 0) return rc;
+    for (int e = 0; e < epochs; ++e) {
+        const std::vector<int32_t>& perm = order[e & 1];
+        HIPCHK(hipMemcpyAsync(m->perm.p, perm.data(), (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
         for (int64_t b = 0; b < nb; ++b) {
-            HIPCHK(launch_gather(m->perm.p + b * batch, batch, m->ds_x.p, m->ds_label.p, m->ds_v.p, m->xb.p, m->lb.p,
-                                 m->vb.p, m->stream));
-            HIPCHK(launch_fill_f32(m->grads.p, 0.0f, kNParams, m->stream));
-            rc = fwd_bwd(m, batch, pos_weight, vel_weight);
-            if (rc) return rc;
             ++m->adam_t;
-            const float bc1 = 1.0f - std::pow(b1, (float)m->adam_t), bc2 = 1.0f - std::pow(b2, (float)m->adam_t);
-            HIPCHK(launch_adam(m->params.p, m->grads.p, m->adam_m.p, m->adam_v.p, kNParams, lr, b1, b2, eps, bc1, bc2,
-                               m->wbf.p, m->stream));
+            t.first = b == 0;
+            t.perm = m->perm.p + b * batch;
+            t.bc1 = 1.0f - std::pow(t.b1, (float)m->adam_t);
+            t.bc2 = 1.0f - std::pow(t.b2, (float)m->adam_t);
+            HIPCHK(launch_train_batch(t, m->stream));
+        }
+        if (e + 1 < epochs) {
+            order[(e + 1) & 1] = perm;
+            shuffle(order[(e + 1) & 1]);
         }
         float L = 0.0f;
-        HIPCHK(hipMemcpyAsync(&L, m->loss.p, sizeof(float), hipMemcpyDeviceToHost, m->stream));
+        HIPCHK(hipMemcpyAsync(&L, t.loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
         HIPCHK(hipStreamSynchronize(m->stream));      // also keeps `perm` alive for the upload
         if (losses) losses[e] = L / (float)nb;
     }

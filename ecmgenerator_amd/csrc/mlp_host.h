@@ -10,28 +10,43 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace ecm {
 namespace mlp {
 
-// feat: [n][8] chunks of 8 BF16 per agent, or with `tiled` chunk c of agent
-// i at ((i / 32) * 8 + c) * 32 + i % 32.
-hipError_t launch_mlp_infer(const void* feat, int tiled, const uint32_t* n_dev, int n_host, const void* frags,
+// in: 0 [n][8] chunks of 8 BF16 per agent, 1 the same tiled (chunk c of agent
+// i at ((i / 32) * 8 + c) * 32 + i % 32), 2 [n][64] FP32.
+hipError_t launch_mlp_infer(const void* feat, int in, const uint32_t* n_dev, int n_host, const void* frags,
                             const float* bias, float theta, uint32_t* mask, float2* vel, float* raw, int n_cu,
                             hipStream_t st);
-hipError_t launch_gemm(int M, int N, int K, const __bf16* A, long sam, long sak, const __bf16* B, long sbn, long sbk,
-                       float* C, long scm, long scn, int accumulate, int splitk, hipStream_t st);
-hipError_t launch_bias_silu(float* Z, const float* bias, __bf16* H, int B, int N, hipStream_t st);
-hipError_t launch_silu_bwd(const float* dH, const float* Z, __bf16* dZ, float* dZf, int B, int N, hipStream_t st);
-hipError_t launch_head(float* Y, const float* bias, const uint32_t* lab, const float2* vt, __bf16* dY, float* dYf,
-                       float* loss, int B, float pos_w, float vel_w, hipStream_t st);
-hipError_t launch_colsum(const float* X, int B, int N, float* out, hipStream_t st);
-hipError_t launch_adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
-                       float bc1, float bc2, __bf16* wb, hipStream_t st);
-hipError_t launch_to_bf16(const float* w, __bf16* wb, int n, hipStream_t st);
-hipError_t launch_f32_to_bf16_rne(const float* x, uint16_t* out, long n, hipStream_t st);
+
+// One batch: forward, backward, gradient and (grad null) one Adam step.
+struct TrainBatch {
+    const int32_t* perm;         // rows of x, label and v, or null: in order
+    const void* x;
+    const uint32_t* label;
+    const float2* v;
+    int n;
+    float pos_w, vel_w;
+    void* frags;                 // [kNTrainFrags][64] packed weights, in and (Adam) out
+    const float* params;
+    void *h[3], *dz[3], *dy;     // [n][128], [n][128], [n][16] BF16
+    float* bias_part;            // [max_blocks][kNBiasParams + 1]
+    int max_blocks;
+    float* part;                 // [train_chunks(n)][kDwFloats]
+    float *w, *m, *v2;
+    float lr, b1, b2, eps, bc1, bc2;
+    float* grad;
+    bool first;                  // the loss of this batch starts the sum
+    float* loss;                 // += the batch's mean loss
+};
+// Batch chunks of the weight gradients: at least 128 rows each, few enough
+// that summing their 172 KB of partial sums stays cheap.
+inline int train_chunks(int n) { return n <= 128 ? 1 : (n >= 96 * 128 ? 96 : (n + 127) / 128); }
+hipError_t launch_train_pack(const float* params, void* frags, hipStream_t st);
+hipError_t launch_train_batch(const TrainBatch& t, hipStream_t st);
 hipError_t launch_fill_f32(float* p, float v, long n, hipStream_t st);
-hipError_t launch_gather(const int64_t* perm, int B, const void* X, const uint32_t* L, const float2* V, void* Xb,
-                         uint32_t* Lb, float2* Vb, hipStream_t st);
 hipError_t launch_pack(const float* P, void* frags, float* bias, hipStream_t st);
 
 }  // namespace mlp
@@ -44,11 +59,11 @@ struct ecm_mlp {
     int dev = 0;
     hipStream_t stream = nullptr;
     int n_cu = 256;
-    // parameters: FP32 master, BF16 row-major copy (training GEMMs),
-    // packed inference fragments and biases
+    // parameters: FP32 master (grads: the gradient, then the loss), packed inference fragments and biases, and
+    // the fragments of a training run (which leaves the others alone)
     ecm::DBuf<float> params, grads, adam_m, adam_v;
-    ecm::DBuf<__bf16> wbf;
-    ecm::DBuf<bf16x8_t> frags;
+    ecm::DBuf<bf16x8_t> frags, tfrags;
+    bool tpacked = false;            // tfrags hold the current parameters
     ecm::DBuf<float> pbias;
     int64_t adam_t = 0;
     // dataset
@@ -57,14 +72,20 @@ struct ecm_mlp {
     ecm::DBuf<float2> ds_v;        // [cap]
     ecm::DBuf<uint32_t> ds_count;  // [1] device append counter
     int64_t ds_cap = 0;
-    // training workspace for batch size ws_batch
-    int ws_batch = 0;
-    ecm::DBuf<int64_t> perm;
+    // BF16 features of the last host batch (kept: a fresh buffer costs a page
+    // fault per 4 KiB in every call)
+    std::vector<uint16_t> h_x;
+    // staged host batch, for batch size in_batch
+    int in_batch = 0;
     ecm::DBuf<bf16x8_t> xb;
     ecm::DBuf<uint32_t> lb;
     ecm::DBuf<float2> vb;
-    ecm::DBuf<float> z1, z2, z3, y, dyf, dh, dzf, loss;
-    ecm::DBuf<__bf16> h1, h2, h3, dy, dz;
+    ecm::DBuf<float> y;
+    // training workspace for batch size ws_batch
+    int ws_batch = 0;
+    ecm::DBuf<int32_t> perm;
+    ecm::DBuf<bf16x8_t> h1, h2, h3, dz1, dz2, dz3, dy;
+    ecm::DBuf<float> part, bias_part;
 };
 
 // Packs the current parameters into the inference layout (stream-ordered).
