@@ -15,11 +15,12 @@
 // bit for bit.
 
 constexpr int kRow = 16;
-// Candidates buffered per agent in the neighbour search: selected down to k
-// (at most 16) when the next 16 would not fit.
-constexpr int kRowCand = 64;
-constexpr int kRowLdsBytes = kRowCand * 12;      // (d2, id) and sorted position of each
-
+// Candidates buffered per agent in the neighbour search, kRowTrip a lane at a
+// time: selected down to k (at most 16) when the next might not fit.
+constexpr int kRowTrip = 4;
+constexpr int kRowCand = 96;
+constexpr int kRowLdsBytes = (kRowCand + 4 + kRow) * 12;      // (d2, id) and sorted position of each candidate, with
+                                                              // room behind them, and of the k selected
 template <int N>
 __device__ __forceinline__ int row_ror(int v) {
     return __builtin_amdgcn_update_dpp(0, v, 0x120 + N, 0xf, 0xf, false);
@@ -212,49 +213,48 @@ __global__ __launch_bounds__(256) void k_scatter_attr_row(DevState s) {
 }
 
 // ------------------------------------------------------------- neighbours
-// One agent's candidates in LDS: (d2, id) pairs and sorted positions.
+// One agent's candidates in LDS, (d2, id) pairs and sorted positions, and the
+// selected ones.
 struct RowCand {
-    float2* di;
-    int* slot;
+    float2 *di, *best;
+    int *slot, *best_slot;
 };
+__device__ __forceinline__ RowCand row_cand(float4* lds) {
+    float2* di = reinterpret_cast<float2*>(lds);
+    int* slot = reinterpret_cast<int*>(di + kRowCand + 4 + kRow);
+    return RowCand{di, di + kRowCand + 4, slot, slot + kRowCand + 4};
+}
 
 // Keeps the k best of the m buffered candidates, in (d2, id) order from
-// entry 0 on: each lane ranks its (up to four) entries against all.
+// entry 0 on: each lane ranks its entries against all, four per trip.
 __device__ __forceinline__ void row_select(const RowCand& B, int k, int l, int& m, float& thr) {
+    // the up to three entries behind the last rank behind every real one
+    if (l < 3) B.di[m + l] = make_float2(INFINITY, __int_as_float(INT_MAX));
     row_fence();
-    float d[4];
-    int id[4], sl[4], rank[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = l + kRow * u;
-        const float2 v = e < m ? B.di[e] : make_float2(INFINITY, 0.0f);
-        d[u] = v.x;
-        id[u] = __float_as_int(v.y);
-        sl[u] = e < m ? B.slot[e] : -1;
-        rank[u] = e < m ? 0 : INT_MAX;
-    }
-    if (m <= kRow) {
-        for (int i = 0; i < m; ++i) {
-            const float2 v = B.di[i];
-            if (rank[0] != INT_MAX) rank[0] += nb_better(v.x, __float_as_int(v.y), d[0], id[0]) ? 1 : 0;
+    const float4* two = reinterpret_cast<const float4*>(B.di);
+    for (int e = l; e - l < m; e += kRow) {
+        const float2 own = e < m ? B.di[e] : make_float2(INFINITY, __int_as_float(INT_MAX));
+        const int id = __float_as_int(own.y);
+        int rank = 0;
+        for (int i = 0; i < m; i += 4) {
+            const float4 a = two[i / 2], b = two[i / 2 + 1];
+            rank += (int)nb_better(a.x, __float_as_int(a.y), own.x, id) +
+                    (int)nb_better(a.z, __float_as_int(a.w), own.x, id) +
+                    (int)nb_better(b.x, __float_as_int(b.y), own.x, id) +
+                    (int)nb_better(b.z, __float_as_int(b.w), own.x, id);
         }
-    } else {
-        for (int i = 0; i < m; ++i) {
-            const float2 v = B.di[i];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (rank[u] != INT_MAX) rank[u] += nb_better(v.x, __float_as_int(v.y), d[u], id[u]) ? 1 : 0;
+        if (e < m && rank < k) {
+            B.best[rank] = own;
+            B.best_slot[rank] = B.slot[e];
         }
     }
-    row_fence();
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-        if (rank[u] < k) {
-            B.di[rank[u]] = make_float2(d[u], __int_as_float(id[u]));
-            B.slot[rank[u]] = sl[u];
-        }
     row_fence();
     m = min(m, k);
+    if (l < m) {
+        B.di[l] = B.best[l];
+        B.slot[l] = B.best_slot[l];
+    }
+    row_fence();
     if (m == k) thr = fminf(thr, B.di[k - 1].x);
 }
 
@@ -263,130 +263,107 @@ __device__ __forceinline__ void row_select(const RowCand& B, int k, int l, int& 
 // is one, else ring by ring until the unvisited region is beyond the k-th),
 // a cell per lane, collected in LDS and ranked by (d2, id).  Returns the
 // count; lane r < count holds the r-th neighbour's sorted position in slot.
-__device__ __forceinline__ int row_knn(const DevState& s, const EnvDesc& E, int t, V2 p, int l, const RowCand& B,
-                                       int& slot) {
+__device__ __forceinline__ int row_knn(const DevState& s, const EnvDesc& E, int t, int q, V2 p, int l,
+                                       const RowCand& B, int& slot) {
     const int k = s.k;
     const GridDesc& g = E.ag;
     float thr = INFINITY;
     {
-        const int q = s.prev_of[t];
-        if (q >= 0 && q < s.n_slots && s.nbr_cnt_prev[q] >= k) {
-            bool ok = true;
-            float d2 = 0.0f;
-            if (l < k) {
-                const int os = s.nbr_prev[(size_t)l * s.n_slots + q];
-                const int f = os >= 0 && os < s.n_slots ? s.fwd[os] : -1;
-                ok = f >= 0 && f < s.n_slots;
-                if (ok) {
-                    const float4 c = s.sorted_pr[f];
-                    const float dx = c.x - p.x, dy = c.y - p.y;
-                    d2 = dx * dx + dy * dy;
-                    ok = d2 > kEps;
-                    if (s.agent_env)
-                        ok &= __float_as_int(s.sorted_v[f].w) == __float_as_int(s.sorted_v[t].w);
-                }
-            }
-            if (row_ballot(!ok) == 0u) thr = row_max(d2);
-        }
+        // the seeds (q: the agent's last sorted position), every level's
+        // loads issued together, out-of-range entries reading entry 0
+        const bool had = q >= 0 && q < s.n_slots;
+        const int had_n = s.nbr_cnt_prev[had ? q : 0];
+        const int os = s.nbr_prev[(size_t)min(l, k - 1) * s.n_slots + (had ? q : 0)];
+        const bool in = os >= 0 && os < s.n_slots;
+        const int f = s.fwd[in ? os : 0];
+        const bool on = in && f >= 0 && f < s.n_slots;
+        const float4 c = s.sorted_pr[on ? f : 0];
+        const float dx = c.x - p.x, dy = c.y - p.y;
+        const float d2 = dx * dx + dy * dy;
+        bool ok = had && had_n >= k && on && d2 > kEps;
+        if (s.agent_env) ok = ok && __float_as_int(s.sorted_v[on ? f : 0].w) == __float_as_int(s.sorted_v[t].w);
+        if (row_ballot(!ok) == 0u) thr = row_max(d2);
     }
     int m = 0;
-    // a cell's agents [a, b) per lane, the lanes in step
-    auto visit = [&](uint32_t a, uint32_t b) {
-        while (row_ballot(a < b)) {
-            bool keep = false;
-            float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            float d2 = 0.0f;
-            if (a < b) {
-                c = s.sorted_pr[a];
-                const float dx = c.x - p.x, dy = c.y - p.y;
-                d2 = dx * dx + dy * dy;
-                keep = d2 > kEps && d2 <= thr;
-            }
-            uint32_t bal = row_ballot(keep);
-            if (m + __popc(bal) > kRowCand) {
-                row_select(B, k, l, m, thr);
-                keep = keep && d2 <= thr;
-                bal = row_ballot(keep);
-            }
-            if (keep) {
-                const int e = m + __popc(bal & ((1u << l) - 1u));
-                B.di[e] = make_float2(d2, c.w);
-                B.slot[e] = (int)a;
-            }
-            m += __popc(bal);
-            ++a;
-        }
-    };
     const float wmax = kKnnWalkCells * g.cell;
-    if (thr <= wmax * wmax) {
-        // every candidate lies in the rectangle of cells around the bound's
-        // circle (knn_query_seeded)
-        const float rr = __fsqrt_rn(thr) * 1.0001f + 2e-3f;
-        const float prune2 = rr * rr;
-        const int xl = grid_cell(p.x - rr, g.x0, g.inv_cell, g.side);
-        const int xh = grid_cell(p.x + rr, g.x0, g.inv_cell, g.side);
-        const int yl = grid_cell(p.y - rr, g.y0, g.inv_cell, g.side);
-        const int yh = grid_cell(p.y + rr, g.y0, g.inv_cell, g.side);
-        const int w = xh - xl + 1, nc = w * (yh - yl + 1);
+    // one rectangle of cells around the bound's circle, which holds every
+    // candidate (knn_query_seeded), or rings around the agent's cell, until
+    // the unvisited region is beyond the k-th (knn_query)
+    const bool rect = thr <= wmax * wmax;
+    const float guard = 2e-3f;
+    int cx = grid_cell(p.x, g.x0, g.inv_cell, g.side);
+    int cy = grid_cell(p.y, g.y0, g.inv_cell, g.side);
+    int w = 1, nc = 1;
+    if (rect) {
+        const float rr = __builtin_amdgcn_sqrtf(thr) * 1.0001f + guard;
+        cx = grid_cell(p.x - rr, g.x0, g.inv_cell, g.side);
+        cy = grid_cell(p.y - rr, g.y0, g.inv_cell, g.side);
+        w = grid_cell(p.x + rr, g.x0, g.inv_cell, g.side) - cx + 1;
+        nc = w * (grid_cell(p.y + rr, g.y0, g.inv_cell, g.side) - cy + 1);
+    }
+    for (int r = 0;; ++r) {
+        if (!rect) nc = r == 0 ? 1 : 8 * r;
+        float prune2 = INFINITY;
+        if (thr < INFINITY) {
+            const float rr = __builtin_amdgcn_sqrtf(thr) * 1.0001f + guard;
+            prune2 = rr * rr;
+        }
         for (int q0 = 0; q0 < nc; q0 += kRow) {
             const int q = q0 + l;
+            int x, y;
+            if (rect) { const int yy = q / w; x = cx + (q - yy * w); y = cy + yy; }
+            else if (r == 0) { x = cx; y = cy; }
+            else if (q < 2 * r + 1) { x = cx - r + q; y = cy + r; }
+            else if (q < 4 * r + 2) { x = cx - r + (q - (2 * r + 1)); y = cy - r; }
+            else if (q < 6 * r + 1) { x = cx - r; y = cy - r + 1 + (q - (4 * r + 2)); }
+            else { x = cx + r; y = cy - r + 1 + (q - (6 * r + 1)); }
             uint32_t a = 0, b = 0;
-            if (q < nc) {
-                const int yy = q / w, x = xl + (q - yy * w), y = yl + yy;
-                if (band_d2(p.x, g.x0, g.cell, x, g.side) + band_d2(p.y, g.y0, g.cell, y, g.side) <= prune2) {
-                    const uint32_t mk_ = E.cell_base + morton2((uint32_t)x, (uint32_t)y);
-                    a = s.cell_start[mk_];
-                    b = s.cell_start[mk_ + 1];
-                }
+            if (q < nc && x >= 0 && y >= 0 && x < g.side && y < g.side &&
+                band_d2(p.x, g.x0, g.cell, x, g.side) + band_d2(p.y, g.y0, g.cell, y, g.side) <= prune2) {
+                const uint32_t key = E.cell_base + morton2((uint32_t)x, (uint32_t)y);
+                a = s.cell_start[key];
+                b = s.cell_start[key + 1];
             }
-            visit(a, b);
-        }
-    } else {
-        // rings around the agent's cell, the perimeter's cells over the lanes
-        const int cx = grid_cell(p.x, g.x0, g.inv_cell, g.side);
-        const int cy = grid_cell(p.y, g.y0, g.inv_cell, g.side);
-        const float guard = 2e-3f;
-        for (int r = 0;; ++r) {
-            const int perim = r == 0 ? 1 : 8 * r;
-            float prune2 = INFINITY;
-            if (thr < INFINITY) {
-                const float rr = __fsqrt_rn(thr) * 1.0001f + guard;
-                prune2 = rr * rr;
-            }
-            for (int q0 = 0; q0 < perim; q0 += kRow) {
-                const int q = q0 + l;
-                uint32_t a = 0, b = 0;
-                if (q < perim) {
-                    int x, y;
-                    if (r == 0) { x = cx; y = cy; }
-                    else if (q < 2 * r + 1) { x = cx - r + q; y = cy + r; }
-                    else if (q < 4 * r + 2) { x = cx - r + (q - (2 * r + 1)); y = cy - r; }
-                    else if (q < 6 * r + 1) { x = cx - r; y = cy - r + 1 + (q - (4 * r + 2)); }
-                    else { x = cx + r; y = cy - r + 1 + (q - (6 * r + 1)); }
-                    if (x >= 0 && y >= 0 && x < g.side && y < g.side &&
-                        band_d2(p.x, g.x0, g.cell, x, g.side) + band_d2(p.y, g.y0, g.cell, y, g.side) <= prune2) {
-                        const uint32_t mk_ = E.cell_base + morton2((uint32_t)x, (uint32_t)y);
-                        a = s.cell_start[mk_];
-                        b = s.cell_start[mk_ + 1];
+            // a cell's agents [a, b) per lane, the lanes in step, kRowTrip at
+            // a time with their loads together
+            while (row_ballot(a < b)) {
+                if (m > kRowCand - kRow * kRowTrip) row_select(B, k, l, m, thr);
+                float4 c[kRowTrip];
+#pragma unroll
+                for (int u = 0; u < kRowTrip; ++u) c[u] = s.sorted_pr[a < b ? min(a + u, b - 1u) : 0u];
+#pragma unroll
+                for (int u = 0; u < kRowTrip; ++u) {
+                    const float dx = c[u].x - p.x, dy = c[u].y - p.y;
+                    const float d2 = dx * dx + dy * dy;
+                    const bool keep = a + u < b && d2 > kEps && d2 <= thr;
+                    const uint32_t bal = row_ballot(keep);
+                    if (keep) {
+                        const int e = m + __popc(bal & ((1u << l) - 1u));
+                        B.di[e] = make_float2(d2, c[u].w);
+                        B.slot[e] = (int)(a + u);
                     }
+                    m += __popc(bal);
                 }
-                visit(a, b);
+                a += kRowTrip;
             }
-            if (m >= k) row_select(B, k, l, m, thr);
-            const int xl = cx - r, xh = cx + r, yl = cy - r, yh = cy + r;
-            if (xl <= 0 && yl <= 0 && xh >= g.side - 1 && yh >= g.side - 1) break;
-            if (thr < INFINITY) {
-                float bnd = INFINITY;
-                if (xl > 0) bnd = fminf(bnd, p.x - (g.x0 + (float)xl * g.cell));
-                if (yl > 0) bnd = fminf(bnd, p.y - (g.y0 + (float)yl * g.cell));
-                if (xh < g.side - 1) bnd = fminf(bnd, (g.x0 + (float)(xh + 1) * g.cell) - p.x);
-                if (yh < g.side - 1) bnd = fminf(bnd, (g.y0 + (float)(yh + 1) * g.cell) - p.y);
-                bnd -= guard;
-                if (bnd > 0.0f && bnd * bnd > thr) break;
+        }
+        const int xl = cx - r, xh = cx + r, yl = cy - r, yh = cy + r;
+        const bool all = rect || (xl <= 0 && yl <= 0 && xh >= g.side - 1 && yh >= g.side - 1);
+        if (all || m >= k) row_select(B, k, l, m, thr);
+        if (all) break;
+        if (thr < INFINITY) {
+            float bnd = INFINITY;
+            if (xl > 0) bnd = fminf(bnd, p.x - (g.x0 + (float)xl * g.cell));
+            if (yl > 0) bnd = fminf(bnd, p.y - (g.y0 + (float)yl * g.cell));
+            if (xh < g.side - 1) bnd = fminf(bnd, (g.x0 + (float)(xh + 1) * g.cell) - p.x);
+            if (yh < g.side - 1) bnd = fminf(bnd, (g.y0 + (float)(yh + 1) * g.cell) - p.y);
+            bnd -= guard;
+            if (bnd > 0.0f && bnd * bnd > thr) {
+                if (m < k) row_select(B, k, l, m, thr);
+                break;
             }
         }
     }
-    row_select(B, k, l, m, thr);
     slot = l < m ? B.slot[l] : -1;
     row_fence();                                     // the buffer is reused
     return m;
@@ -523,12 +500,33 @@ __device__ __forceinline__ void row_lp3d(const RowList& C, V2 an, V2 ap, float m
     }
 }
 
+// The obstacle edge of a lane: its loads, apart from its constraint.
+struct RowEdge {
+    int e;                    // -1: none
+    float4 a, b;
+    uint8_t fl;
+};
+__device__ __forceinline__ RowEdge row_edge(const EnvDesc& E, int q, int e1) {
+    RowEdge r;
+    r.e = q < e1 ? E.obucket_edges[q] : -1;
+    const int at = max(r.e, 0);
+    r.a = E.oe0[at];
+    r.b = E.oe1[at];
+    r.fl = E.oflags[at];
+    return r;
+}
+
 // Neighbour search, ORCA, both LPs and the integration of the agent at
 // sorted position t.  lds: the row's share, room for maxo obstacle
-// constraints and for the candidate buffer (used one after the other).
+// constraints and for the candidate buffer (used one after the other).  The
+// loads of the obstacle edges go out before the neighbour search and those
+// of the neighbours before the edges' half-planes: a lone wavefront waits for
+// each level of dependent loads, 500-900 cycles, and there are a dozen.
 __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, float4* lds, int maxo) {
     const float4 pr = s.sorted_pr[t];
     const float4 sv = s.sorted_v[t];
+    const int prev = s.prev_of[t];
+    const float2 pv = s.pref_vel_s[t];
     if (s.dead_s[t]) {                               // destroyed this step: state unchanged
         if (l == 0) {
             s.nbr_cnt[t] = 0;
@@ -542,9 +540,18 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
     const float rad = pr.z;
     const float maxSpeed = s.max_speed_from_pref ? sv.z : s.max_speed;
     const EnvDesc& E = env_of_sorted(s, sv);
+    const bool obst = E.n_obst_edges > 0;
+    int e0 = 0, e1 = 0;
+    RowEdge edge;
+    if (obst) {
+        obstacle_bucket(E, position, e0, e1);
+        edge = row_edge(E, e0 + l, e1);
+    }
     int slot;
-    const RowCand B{reinterpret_cast<float2*>(lds), reinterpret_cast<int*>(lds) + 2 * kRowCand};
-    const int cnt = row_knn(s, E, t, position, l, B, slot);
+    const RowCand B = row_cand(lds);
+    const int cnt = row_knn(s, E, t, prev, position, l, B, slot);
+    const float4 q = s.sorted_pr[l < cnt ? slot : t];
+    const float2 qv = sorted_vel(s, l < cnt ? slot : t);
     if (l < cnt) s.nbr[(size_t)l * s.n_slots + t] = slot;
     if (l == 0) s.nbr_cnt[t] = cnt;
 
@@ -553,18 +560,15 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
     C.nO = 0;
     C.na = cnt;
     // the edges of the bucket, one per lane, kept in bucket order
-    if (E.n_obst_edges > 0) {
+    if (obst) {
         const float range = s.time_horizon_obst * maxSpeed + rad;          // ORCA.cpp:27
-        int e0, e1;
-        obstacle_bucket(E, position, e0, e1);
         for (int q0 = e0; q0 < e1; q0 += kRow) {
-            const int q = q0 + l;
+            if (q0 > e0) edge = row_edge(E, q0 + l, e1);
             bool made = false;
             V2 cp = mk(0.0f, 0.0f), cn = mk(0.0f, 0.0f);
-            int e;
             float dd;
-            if (q < e1 && obstacle_near(E, position, range * range, q, e, dd))
-                made = obstacle_constraint(s, E, e, position, velocity, rad, cp, cn);
+            if (edge.e >= 0 && edge_near(edge.a, position, range * range, dd))
+                made = edge_constraint(s, edge.a, edge.b, edge.fl, position, velocity, rad, cp, cn);
             const uint32_t m = row_ballot(made);
             const int at = C.nO + __popc(m & ((1u << l) - 1u));
             if (made && at < maxo) lds[at] = make_float4(cn.x, cn.y, cp.x, cp.y);
@@ -573,12 +577,12 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
         C.nO = min(C.nO, maxo);                      // maxo covers the longest bucket
     }
     V2 an = mk(0.0f, 0.0f), ap = mk(0.0f, 0.0f);
-    if (l < cnt) agent_constraint(s, position, velocity, rad, s.sorted_pr[slot], sorted_vel(s, slot), ap, an);
+    if (l < cnt && !(s.inv_dt != 0.0f && agent_constraint_common(s, position, velocity, rad, q, qv, ap, an)))
+        agent_constraint(s, position, velocity, rad, q, qv, ap, an);
     row_fence();
     const float4 own = l < C.nO ? lds[l] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     C.on = ob_n(own);
     C.op = ob_p(own);
-    const float2 pv = s.pref_vel_s[t];
     V2 o;
     const int n = C.nO + cnt;
     const int fail = row_lp<false>(C, an, ap, (1u << cnt) - 1u, mk(pv.x, pv.y), maxSpeed, l, o);
@@ -593,7 +597,7 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
 }
 
 // One wavefront per block: four agents at a time, strided over the grid.
-__global__ __launch_bounds__(64) void k_row_step(DevState s, int maxo, int row_f4) {
+__global__ __launch_bounds__(64, 5) void k_row_step(DevState s, int maxo, int row_f4) {
     extern __shared__ float4 row_lds[];
     const int n_active = (int)s.cell_start[s.n_keys];
     const int r = threadIdx.x / kRow, l = threadIdx.x & (kRow - 1);

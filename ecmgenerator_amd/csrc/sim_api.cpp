@@ -36,7 +36,7 @@ hipError_t launch_mark_dead(const int* ids, int n, const int* pos_of, const floa
                             const unsigned long long* acc, hipStream_t st);
 hipError_t launch_knn(const DevState& s, int block, int mode, int oslots, hipStream_t st);
 hipError_t launch_orca(const DevState& s, int maxo, int mode, int oslots, int n_cu, hipStream_t st, hipEvent_t mid);
-hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st);
+hipError_t launch_row_step(const DevState& s, int maxo, int agents, hipStream_t st);
 hipError_t launch_features(const DevState& s, hipStream_t st);
 hipError_t launch_export_nbrs(const DevState& s, int* out, int* out_cnt, hipStream_t st);
 hipError_t launch_spawn_scatter(int n, const int* ids, const float2* start, const float* rad, const float* spd,
@@ -265,7 +265,7 @@ struct ecm_sim {
     // recaptured when anything they were captured with changes
     struct GraphKey {
         DevState d;
-        int maxo, mode, oslots, knn_block, n_cu, row;
+        int maxo, mode, oslots, knn_block, n_cu, row, row_agents;
         float theta;
         const void* frags;
         const void* pbias;
@@ -279,6 +279,7 @@ struct ecm_sim {
     bool use_graph = false;
     bool idle = true;                           // nothing queued on the stream since it was last waited for
     bool row_step = false, row_attr = false;    // 16 lanes per agent (row_rule)
+    int row_agents = 0;                         // agents their grid is sized for
     StepGraph graphs[2][2];                     // [parity][entry from the sorted outputs]
     std::string graph_error;
     std::vector<int> h_replans;
@@ -1392,6 +1393,10 @@ static DevState make_state(ecm_sim* s) {
         const float inv = 1.0f / s->prm.time_horizon;
         d.inv_time_horizon = (m == 0.5f && std::isnormal(inv) && inv * s->prm.time_horizon == 1.0f) ? inv : 0.0f;
     }
+    {
+        auto within = [](float v) { return v >= 0x1p-20f && v <= 0x1p20f; };
+        d.inv_dt = d.inv_time_horizon != 0.0f && within(s->prm.time_horizon) && within(s->prm.dt) ? 1.0f / s->prm.dt : 0.0f;
+    }
     d.time_horizon_obst = s->prm.time_horizon_obst;
     d.inv_time_horizon_obst = 1.0f / s->prm.time_horizon_obst;
     d.max_speed = s->prm.max_speed;
@@ -1569,6 +1574,7 @@ static void row_rule(ecm_sim* s, int mode) {
     const bool shape = mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2;
     s->row_step = shape && small(s->row_step, kRowAgents);
     s->row_attr = shape && small(s->row_attr, kRowAttrAgents);
+    s->row_agents = s->row_step ? (s->num_agents + 4095) / 4096 * 4096 : 0;
 }
 
 static int step_mode(const ecm_sim* s) { return s->log_mlp ? 1 : (s->mlp ? 2 : 0); }
@@ -1588,7 +1594,7 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
         if (s->timing) HIPCHK(hipEventRecord(s->ev[6], s->stream));
         // the plain step's main ORCA pass may run inside the k-nearest
         // kernel, or the whole rest of the step in one kernel
-        if (s->row_step) HIPCHK(launch_row_step(d, s->maxo, s->n_cu, s->stream));
+        if (s->row_step) HIPCHK(launch_row_step(d, s->maxo, s->row_agents, s->stream));
         else HIPCHK(launch_knn(d, s->tune.knn_block, mode, s->tune.orca_obst_slots, s->stream));
         return 0;
     }
@@ -1657,6 +1663,7 @@ static int ensure_step_graph(ecm_sim* s, const DevState& d, int mode) {
     key.frags = mode == 2 ? (const void*)s->mlp->frags.p : nullptr;
     key.pbias = mode == 2 ? (const void*)s->mlp->pbias.p : nullptr;
     key.n_cu = mode == 2 ? s->mlp->n_cu : 0;
+    key.row_agents = s->row_agents;
     key.row = (s->row_step ? 1 : 0) | (s->row_attr ? 2 : 0);
     ecm_sim::StepGraph& g = s->graphs[s->cur][d.sorted_in];
     if (g.valid && std::memcmp(&g.key, &key, sizeof(key)) == 0) return 0;

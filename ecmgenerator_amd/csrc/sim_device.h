@@ -169,6 +169,8 @@ struct DevState {
     int k;
     float time_horizon;
     float inv_time_horizon;       // 1 / time_horizon when that is exact (a power of two), else 0
+    float inv_dt;                 // 1 / dt when T is a power of two and both are in [2^-20, 2^20] (then
+                                  // agent_constraint_common applies), else 0
     float time_horizon_obst;
     float inv_time_horizon_obst;  // 1.0f / time_horizon_obst (ORCA.cpp:241)
     float max_speed;

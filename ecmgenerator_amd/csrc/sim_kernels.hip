@@ -1033,12 +1033,11 @@ __device__ __forceinline__ float4* q3d_slot(const DevState& s, uint32_t q, int c
 // Constraint::Contains, methodB (ORCA.h:49-60)
 __device__ __forceinline__ bool con_contains(const Con& c, V2 q) { return det(right(c.n), c.p - q) <= 0.0f; }
 
-// Obstacle half-plane for edge e (ORCA.cpp:70-333).  Returns false when the
-// reference emits nothing for it (`continue` without push_back).
-__device__ bool obstacle_constraint(const DevState& s, const EnvDesc& E, int e, V2 position, V2 velocity, float rad,
-                                    V2& outP, V2& outN) {
-    float4 a = E.oe0[e], b = E.oe1[e];
-    uint8_t fl = E.oflags[e];
+// Obstacle half-plane for an edge (its oe0, oe1 and oflags; ORCA.cpp:70-333).
+// Returns false when the reference emits nothing for it (`continue` without
+// push_back).
+__device__ bool edge_constraint(const DevState& s, float4 a, float4 b, uint8_t fl, V2 position, V2 velocity, float rad,
+                                V2& outP, V2& outN) {
     V2 pL = mk(a.x, a.y), pR = mk(a.z, a.w);
     V2 pPrevL = mk(b.x, b.y), pNextR = mk(b.z, b.w);
     bool cvL = fl & 1, cvR = (fl >> 1) & 1;
@@ -1147,6 +1146,11 @@ __device__ bool obstacle_constraint(const DevState& s, const EnvDesc& E, int e, 
     }
 }
 
+__device__ __forceinline__ bool obstacle_constraint(const DevState& s, const EnvDesc& E, int e, V2 position, V2 velocity,
+                                                    float rad, V2& outP, V2& outN) {
+    return edge_constraint(s, E.oe0[e], E.oe1[e], E.oflags[e], position, velocity, rad, outP, outN);
+}
+
 // Agent half-plane (ORCA.cpp:339-423)
 __device__ void agent_constraint(const DevState& s, V2 position, V2 velocity, float rad,
                                  float4 q, float2 qv, V2& outP, V2& outN) {
@@ -1195,6 +1199,51 @@ __device__ void agent_constraint(const DevState& s, V2 position, V2 velocity, fl
             outP = velocity + U * 0.5f; outN = right(rl);
         }
     }
+}
+
+// agent_constraint without a branch, for the common operands: false where one
+// of them is outside the ranges of the cheap quotients (tiny, huge or NaN
+// coordinates, the side of a leg within rounding), and the caller takes
+// agent_constraint then.  Needs s.inv_dt.  The three kinds (colliding, on the
+// cutoff disc, on a leg) each normalise one vector: it is selected first and
+// normalised once.  With T a power of two the scaled length is the length
+// scaled, so one root serves both, and the legs' angle is that of the
+// unscaled radius and distance.  About 170 instructions against 330 in a
+// wavefront whose lanes meet every kind.
+__device__ __forceinline__ bool agent_constraint_common(const DevState& s, V2 position, V2 velocity, float rad,
+                                                        float4 q, float2 qv, V2& outP, V2& outN) {
+    const float combined = q.z + rad;
+    const V2 relVel = mk(velocity.x - qv.x, velocity.y - qv.y);
+    const V2 relPos = mk(q.x - position.x, q.y - position.y);
+    const float S = len2(relPos);
+    const float y = __builtin_amdgcn_rsqf(S);
+    const float l = root_from(S, y);
+    const bool colliding = l < combined;
+    const V2 VOPos = relPos * s.inv_time_horizon;
+    V2 left_leg, right_leg;
+    rotate_pm(VOPos, atan_unit(quot(combined, l, recip_from(l, y))), left_leg, right_leg);
+    const V2 w = relVel - VOPos;
+    const bool below = det(left_leg - VOPos, w) > 0;
+    // sign of dot(left(VOPos) / |VOPos|, relVel): that of the undivided
+    // product, unless it is within the rounding of the divided one
+    const float c0 = VOPos.y * relVel.x, c1 = VOPos.x * relVel.y, side = c1 - c0;
+    const bool sure = fabsf(side) > __builtin_fmaf(0x1p-20f, fabsf(c0) + fabsf(c1), 0x1p-60f);
+    const bool on_left = side > 0.0f, disc = colliding || below;
+    const V2 wc = relVel - quot(relPos, s.dt, s.inv_dt);
+    const V2 leg = mk(on_left ? left_leg.x : right_leg.x, on_left ? left_leg.y : right_leg.y);
+    const V2 v = mk(colliding ? wc.x : (below ? w.x : leg.x), colliding ? wc.y : (below ? w.y : leg.y));
+    const float R = colliding ? quot(combined, s.dt, s.inv_dt) : combined * s.inv_time_horizon;
+    const float Sv = len2(v);
+    const float yv = __builtin_amdgcn_rsqf(Sv);
+    const float lv = root_from(Sv, yv);
+    const V2 u = quot(v, lv, recip_from(lv, yv));
+    const float f = disc ? R - lv : dot(relVel, u);
+    V2 U = u * f;
+    U = mk(disc ? U.x : U.x - relVel.x, disc ? U.y : U.y - relVel.y);
+    outP = velocity + U * 0.5f;
+    outN = mk(disc ? u.x : (on_left ? -u.y : u.y), disc ? u.y : (on_left ? u.x : -u.x));
+    return exp_within(S, -60, 60) & exp_within(combined, -60, 60) & not_tiny(relPos) & !all_ones(l) &
+           exp_within(Sv, -60, 60) & not_tiny(v) & !all_ones(lv) & (disc | sure);
 }
 
 // ORCA::RandomizedLP (ORCA.cpp:428-587) over a virtual list: entries
@@ -1370,13 +1419,10 @@ __device__ __forceinline__ void obstacle_bucket(const EnvDesc& s, V2 position, i
     e0 = s.obucket_start[b];
     e1 = s.obucket_start[b + 1];
 }
-// Whether bucket entry q is an obstacle neighbour of position (the test of
-// Simulator.cpp:266-287); e receives its edge, dd the squared distance to
-// the edge's closest point.
-__device__ __forceinline__ bool obstacle_near(const EnvDesc& s, V2 position, float range2, int q, int& e,
-                                              float& dd) {
-    e = s.obucket_edges[q];
-    float4 a = s.oe0[e];
+// Whether an edge (its oe0) is an obstacle neighbour of position (the test of
+// Simulator.cpp:266-287); dd receives the squared distance to its closest
+// point.
+__device__ __forceinline__ bool edge_near(float4 a, V2 position, float range2, float& dd) {
     V2 L = mk(a.x, a.y), R = mk(a.z, a.w);
     float sld = det(L - position, R - L);
     float sqd = sld * sld / sq_dist(L, R);
@@ -1384,6 +1430,12 @@ __device__ __forceinline__ bool obstacle_near(const EnvDesc& s, V2 position, flo
     V2 c = closest_on_segment(position, L, R);
     dd = sq_dist(c, position);
     return dd < range2;
+}
+// The same for bucket entry q; e receives its edge.
+__device__ __forceinline__ bool obstacle_near(const EnvDesc& s, V2 position, float range2, int q, int& e,
+                                              float& dd) {
+    e = s.obucket_edges[q];
+    return edge_near(s.oe0[e], position, range2, dd);
 }
 // Obstacle query with the reference's filter (Simulator.cpp:266-287) over
 // the agent's bucket; `emit(e, dd)` runs for every edge it keeps, in scan
@@ -2199,11 +2251,11 @@ static void launch_orca_k(const DevState& s, int maxo, int mode, int oslots, int
 }
 
 // The neighbour search and ORCA with 16 lanes per agent (row_kernels.h): the
-// rest of the plain step.  A grid of at most 32 wavefronts per CU, strided,
-// so that spare slots of a large pool cost nothing.
-hipError_t launch_row_step(const DevState& s, int maxo, int n_cu, hipStream_t st) {
+// rest of the plain step.  A wavefront for every four of `agents` (the kernel
+// strides, so that any count is covered).
+hipError_t launch_row_step(const DevState& s, int maxo, int agents, hipStream_t st) {
     const int row_f4 = std::max(maxo, kRowLdsBytes / 16);
-    hipLaunchKernelGGL(k_row_step, dim3(std::min(round8(cdiv(s.n_slots, 4)), round8(std::max(1, n_cu) * 32))), dim3(64),
+    hipLaunchKernelGGL(k_row_step, dim3(round8(cdiv(std::max(1, std::min(agents, s.n_slots)), 4))), dim3(64),
                        (size_t)row_f4 * 4 * sizeof(float4), st, s, maxo, row_f4);
     return hipGetLastError();
 }
