@@ -23,23 +23,24 @@ constexpr int kRowLdsBytes = (kRowCand + 4 + kRow) * 12;      // (d2, id) and so
                                                               // room behind them, and of the k selected
 template <int N>
 __device__ __forceinline__ int row_ror(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, 0x120 + N, 0xf, 0xf, false);
+    return __builtin_amdgcn_mov_dpp(v, 0x120 + N, 0xf, 0xf, true);
 }
-template <int N>
-__device__ __forceinline__ float row_ror(float v) { return __int_as_float(row_ror<N>(__float_as_int(v))); }
 // Reductions over the 16 lanes, the result in every lane.
-__device__ __forceinline__ float row_min(float v) {
-    v = fminf(v, row_ror<8>(v)); v = fminf(v, row_ror<4>(v)); v = fminf(v, row_ror<2>(v));
-    return fminf(v, row_ror<1>(v));
-}
-__device__ __forceinline__ float row_max(float v) {
-    v = fmaxf(v, row_ror<8>(v)); v = fmaxf(v, row_ror<4>(v)); v = fmaxf(v, row_ror<2>(v));
-    return fmaxf(v, row_ror<1>(v));
-}
 __device__ __forceinline__ int row_min(int v) {
     v = min(v, row_ror<8>(v)); v = min(v, row_ror<4>(v)); v = min(v, row_ror<2>(v));
     return min(v, row_ror<1>(v));
 }
+__device__ __forceinline__ int row_max(int v) {
+    v = max(v, row_ror<8>(v)); v = max(v, row_ror<4>(v)); v = max(v, row_ror<2>(v));
+    return max(v, row_ror<1>(v));
+}
+// Floats (no NaN) as integers of the same order, and back: the integer
+// minimum takes one DPP instruction a step, the float one also quiets.
+__device__ __forceinline__ int order_of(float v) {
+    const int b = __float_as_int(v);
+    return b ^ ((b >> 31) & 0x7fffffff);
+}
+__device__ __forceinline__ float of_order(int v) { return __int_as_float(v ^ ((v >> 31) & 0x7fffffff)); }
 // The row's bits of the wavefront's ballot.
 __device__ __forceinline__ uint32_t row_ballot(bool b) {
     return (uint32_t)(__ballot(b) >> (__lane_id() & 48u)) & 0xffffu;
@@ -282,7 +283,7 @@ __device__ __forceinline__ int row_knn(const DevState& s, const EnvDesc& E, int 
         const float d2 = dx * dx + dy * dy;
         bool ok = had && had_n >= k && on && d2 > kEps;
         if (s.agent_env) ok = ok && __float_as_int(s.sorted_v[on ? f : 0].w) == __float_as_int(s.sorted_v[t].w);
-        if (row_ballot(!ok) == 0u) thr = row_max(d2);
+        if (row_ballot(!ok) == 0u) thr = __int_as_float(row_max(__float_as_int(d2)));       // d2 > 0
     }
     int m = 0;
     const float wmax = kKnnWalkCells * g.cell;
@@ -301,6 +302,9 @@ __device__ __forceinline__ int row_knn(const DevState& s, const EnvDesc& E, int 
         w = grid_cell(p.x + rr, g.x0, g.inv_cell, g.side) - cx + 1;
         nc = w * (grid_cell(p.y + rr, g.y0, g.inv_cell, g.side) - cy + 1);
     }
+    // q / w for the rectangle's few hundred cells: half a cell from any
+    // whole quotient, far more than the reciprocal's error
+    const float inv_w = __builtin_amdgcn_rcpf((float)w);
     for (int r = 0;; ++r) {
         if (!rect) nc = r == 0 ? 1 : 8 * r;
         float prune2 = INFINITY;
@@ -311,7 +315,7 @@ __device__ __forceinline__ int row_knn(const DevState& s, const EnvDesc& E, int 
         for (int q0 = 0; q0 < nc; q0 += kRow) {
             const int q = q0 + l;
             int x, y;
-            if (rect) { const int yy = q / w; x = cx + (q - yy * w); y = cy + yy; }
+            if (rect) { const int yy = (int)(((float)q + 0.5f) * inv_w); x = cx + (q - yy * w); y = cy + yy; }
             else if (r == 0) { x = cx; y = cy; }
             else if (q < 2 * r + 1) { x = cx - r + q; y = cy + r; }
             else if (q < 4 * r + 2) { x = cx - r + (q - (2 * r + 1)); y = cy - r; }
@@ -372,9 +376,10 @@ __device__ __forceinline__ int row_knn(const DevState& s, const EnvDesc& E, int 
 // -------------------------------------------------------------------- LPs
 // A row's constraint list in the reference's order: nO obstacle constraints
 // in LDS (ob, the first 16 also in on / op of lane c), then na agent
-// constraints, number a in an / ap of lane a.
+// constraints, number a in an / ap of lane a; pool is LDS for 16 of those.
 struct RowList {
     const float4* ob;
+    float4* pool;
     int nO, na;
     V2 on, op;
 };
@@ -382,22 +387,28 @@ struct RowList {
 __device__ __forceinline__ V2 ob_n(const float4& c) { return mk(c.x, c.y); }
 __device__ __forceinline__ V2 ob_p(const float4& c) { return mk(c.z, c.w); }
 
-// The first constraint from index i on that `test` holds for, or nO + na;
-// agent constraints outside the bits of aval are passed over.
+// The first constraint from index i < nO + na on that `test` holds for, or
+// nO + na; agent constraints outside the bits of aval are passed over.
 template <typename F>
 __device__ __forceinline__ int row_first(const RowList& C, V2 an, V2 ap, uint32_t aval, int i, int l, F&& test) {
+    const bool va = ((aval >> l) & 1u) && test(an, ap);
+    if (C.nO <= kRow) {
+        // both of a lane's constraints at once
+        const bool vo = l < C.nO && test(C.on, C.op);
+        const uint32_t m = (row_ballot(vo) | (row_ballot(va) << C.nO)) & (~0u << i);
+        return m ? __ffs((int)m) - 1 : C.nO + C.na;
+    }
     for (int c0 = i & ~(kRow - 1); c0 < C.nO; c0 += kRow) {
         const int c = c0 + l;
         bool v = false;
         if (c >= i && c < C.nO) {
-            V2 n = C.on, p = C.op;
-            if (c0 > 0) { const float4 q = C.ob[c]; n = ob_n(q); p = ob_p(q); }
-            v = test(n, p);
+            const float4 q = C.ob[c];
+            v = test(ob_n(q), ob_p(q));
         }
         const uint32_t m = row_ballot(v);
         if (m) return c0 + __ffs((int)m) - 1;
     }
-    const uint32_t m = row_ballot(l >= i - C.nO && ((aval >> l) & 1u) && test(an, ap));
+    const uint32_t m = row_ballot(va && l >= i - C.nO);
     return m ? C.nO + __ffs((int)m) - 1 : C.nO + C.na;
 }
 
@@ -413,19 +424,20 @@ __device__ __forceinline__ int row_lp(const RowList& C, V2 an, V2 ap, uint32_t a
     if (DIR) out = opt * maxSpeed;
     else if (len(opt) > maxSpeed) out = normalized(opt) * maxSpeed;
     else out = opt;
+    C.pool[l] = make_float4(an.x, an.y, ap.x, ap.y);
+    row_fence();
     const int n = C.nO + C.na;
     int i = 0;
-    while (true) {
+    while (i < n) {
         i = row_first(C, an, ap, aval, i, l, [&](V2 cn, V2 cp) { return !(det(right(cn), cp - out) <= 0.0f); });
         if (i >= n) return n;
-        V2 hn, hp;
-        if (i < C.nO) { const float4 q = C.ob[i]; hn = ob_n(q); hp = ob_p(q); }
-        else { hn = row_get(an, i - C.nO); hp = row_get(ap, i - C.nO); }
+        const float4 h = *(i < C.nO ? C.ob + i : C.pool + (i - C.nO));
+        const V2 hn = ob_n(h), hp = ob_p(h);
         const V2 dir = right(hn);
         const float dpd = dot(dir, hp);
         const float disc = dpd * dpd + maxSpeed * maxSpeed - dot(hp, hp);
         if (disc <= 0.0f) return i;
-        const float sq = sqrtf(disc);
+        const float sq = exp_within(disc, -96, 96) ? root_from(disc, __builtin_amdgcn_rsqf(disc)) : sqrtf(disc);
         float lo = -INFINITY, hi = INFINITY;
         int klo = INT_MAX, khi = INT_MAX;           // 2 index + sign of the lane's bound
         bool bad = false;
@@ -446,20 +458,25 @@ __device__ __forceinline__ int row_lp(const RowList& C, V2 an, V2 ap, uint32_t a
         for (int c = l + kRow; c < oi; c += kRow) { const float4 q = C.ob[c]; narrow(c, ob_n(q), ob_p(q)); }
         if (l < i - C.nO && ((aval >> l) & 1u)) narrow(C.nO + l, an, ap);
         if (row_ballot(bad)) return i;
-        float tl = row_max(lo), tr = row_min(hi);
-        if (tl == 0.0f) tl = row_min(lo == 0.0f ? klo : INT_MAX) & 1 ? -0.0f : 0.0f;
-        if (tr == 0.0f) tr = row_min(hi == 0.0f ? khi : INT_MAX) & 1 ? -0.0f : 0.0f;
+        float tl = of_order(row_max(order_of(lo))), tr = of_order(row_min(order_of(hi)));
+        if (tl == 0.0f || tr == 0.0f) {
+            if (tl == 0.0f) tl = row_min(lo == 0.0f ? klo : INT_MAX) & 1 ? -0.0f : 0.0f;
+            if (tr == 0.0f) tr = row_min(hi == 0.0f ? khi : INT_MAX) & 1 ? -0.0f : 0.0f;
+        }
         const float lft = std_max(-dpd - sq, tl);
         const float rgt = std_min(-dpd + sq, tr);
         if (lft > rgt) return i;
+        float t;
         if (DIR) {
-            out = dot(opt, dir) > 0 ? hp + dir * rgt : hp + dir * lft;
+            t = dot(opt, dir) > 0 ? rgt : lft;
         } else {
-            const float t = dot(dir, opt - hp);
-            out = t < lft ? hp + dir * lft : (t > rgt ? hp + dir * rgt : hp + dir * t);
+            t = dot(dir, opt - hp);
+            t = t < lft ? lft : (t > rgt ? rgt : t);
         }
+        out = hp + dir * t;
         ++i;
     }
+    return n;
 }
 
 // RandomizedLP3D (ORCA.cpp:592-669): the bisectors with the agent
@@ -469,7 +486,7 @@ __device__ __forceinline__ void row_lp3d(const RowList& C, V2 an, V2 ap, float m
     const uint32_t all = (1u << C.na) - 1u;
     float maxPen = 0.0f;
     int i = failed;
-    while (true) {
+    while (i < n) {
         i = row_first(C, an, ap, all, i, l, [&](V2 cn, V2 cp) { return !(det(right(cn), cp - out) <= maxPen); });
         if (i >= n) return;
         V2 cn, cp;
@@ -503,8 +520,7 @@ __device__ __forceinline__ void row_lp3d(const RowList& C, V2 an, V2 ap, float m
 // The obstacle edge of a lane: its loads, apart from its constraint.
 struct RowEdge {
     int e;                    // -1: none
-    float4 a, b;
-    uint8_t fl;
+    float4 a, b, c;
 };
 __device__ __forceinline__ RowEdge row_edge(const EnvDesc& E, int q, int e1) {
     RowEdge r;
@@ -512,13 +528,13 @@ __device__ __forceinline__ RowEdge row_edge(const EnvDesc& E, int q, int e1) {
     const int at = max(r.e, 0);
     r.a = E.oe0[at];
     r.b = E.oe1[at];
-    r.fl = E.oflags[at];
+    r.c = E.oe2[at];
     return r;
 }
 
 // Neighbour search, ORCA, both LPs and the integration of the agent at
-// sorted position t.  lds: the row's share, room for maxo obstacle
-// constraints and for the candidate buffer (used one after the other).  The
+// sorted position t.  lds: the row's share, room for maxo obstacle and 16
+// agent constraints and for the candidate buffer (used one after the other).  The
 // loads of the obstacle edges go out before the neighbour search and those
 // of the neighbours before the edges' half-planes: a lone wavefront waits for
 // each level of dependent loads, 500-900 cycles, and there are a dozen.
@@ -557,6 +573,7 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
 
     RowList C;
     C.ob = lds;
+    C.pool = lds + maxo;
     C.nO = 0;
     C.na = cnt;
     // the edges of the bucket, one per lane, kept in bucket order
@@ -568,7 +585,7 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
             V2 cp = mk(0.0f, 0.0f), cn = mk(0.0f, 0.0f);
             float dd;
             if (edge.e >= 0 && edge_near(edge.a, position, range * range, dd))
-                made = edge_constraint(s, edge.a, edge.b, edge.fl, position, velocity, rad, cp, cn);
+                made = edge_constraint(s, edge.a, edge.b, edge.c, position, velocity, rad, cp, cn);
             const uint32_t m = row_ballot(made);
             const int at = C.nO + __popc(m & ((1u << l) - 1u));
             if (made && at < maxo) lds[at] = make_float4(cn.x, cn.y, cp.x, cp.y);

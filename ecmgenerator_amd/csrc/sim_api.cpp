@@ -104,8 +104,7 @@ struct EnvHost {
     std::vector<float> obs_xy;
     std::vector<int> obs_ring_off;
     int n_obst_edges = 0;
-    DBuf<float4> oe0, oe1;
-    DBuf<uint8_t> oflags;
+    DBuf<float4> oe0, oe1, oe2;
     GridDesc og{};
     DBuf<int> obucket_start, obucket_edges;
     int maxo = 16;
@@ -131,7 +130,7 @@ struct EnvHost {
     ecm_replan_fn replan_fn = nullptr;
     void* replan_user = nullptr;
     void release() {
-        oe0.release(); oe1.release(); oflags.release(); obucket_start.release(); obucket_edges.release();
+        oe0.release(); oe1.release(); oe2.release(); obucket_start.release(); obucket_edges.release();
         cellA.release(); cellB.release(); ebucket_start.release(); ebucket_cells.release();
         yhash_key.release(); yhash_off.release(); yhash_cnt.release(); ycells.release();
     }
@@ -640,8 +639,7 @@ extern "C" int ecm_sim_env_set_obstacles(ecm_sim* s, int env, const float* xy, c
     if (nv == 0) { E->obst_range_built = -1.0f; s->envs_dirty = true; return 0; }
     // Obstacle::Initialize (ECMDataTypes.cpp:23-61): prev/next in the ring,
     // isConvex = det(prev - next, p - prev) >= 0 (true for 2-vertex rings).
-    std::vector<float4> e0(nv), e1(nv);
-    std::vector<uint8_t> fl(nv);
+    std::vector<float4> e0(nv), e1(nv), e2(nv);
     std::vector<uint8_t> convex(nv);
     std::vector<int> nxt(nv), prv(nv);
     for (int r = 0; r < n_rings; ++r) {
@@ -660,19 +658,24 @@ extern "C" int ecm_sim_env_set_obstacles(ecm_sim* s, int env, const float* xy, c
             convex[v] = det(A - B, P - A) >= 0.0f;
         }
     }
+    // what an edge's half-plane takes from the edge alone, in the arithmetic
+    // the kernels use (correctly rounded on both sides)
     for (int v = 0; v < nv; ++v) {
-        int R = nxt[v];
+        const int R = nxt[v];
+        auto pt = [&](int i) { return mk(xy[2 * i], xy[2 * i + 1]); };
+        const V2 seg = pt(R) - pt(v), us = normalize(seg), ul = normalize(pt(v) - pt(prv[v])), ur = normalize(pt(nxt[R]) - pt(R));
+        const int fl = convex[v] | (convex[R] << 1);
         e0[v] = make_float4(xy[2 * v], xy[2 * v + 1], xy[2 * R], xy[2 * R + 1]);
-        e1[v] = make_float4(xy[2 * prv[v]], xy[2 * prv[v] + 1], xy[2 * nxt[R]], xy[2 * nxt[R] + 1]);
-        fl[v] = (uint8_t)(convex[v] | (convex[R] << 1));
+        e1[v] = make_float4(ul.x, ul.y, ur.x, ur.y);
+        e2[v] = make_float4(us.x, us.y, len2(seg), bits_to_float(fl));
     }
     int rc = E->oe0.alloc(nv);
     if (!rc) rc = E->oe1.alloc(nv);
-    if (!rc) rc = E->oflags.alloc(nv);
+    if (!rc) rc = E->oe2.alloc(nv);
     if (rc) return rc;
     HIPCHK(hipMemcpyAsync(E->oe0.p, e0.data(), nv * sizeof(float4), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(E->oe1.p, e1.data(), nv * sizeof(float4), hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipMemcpyAsync(E->oflags.p, fl.data(), nv, hipMemcpyHostToDevice, s->stream));
+    HIPCHK(hipMemcpyAsync(E->oe2.p, e2.data(), nv * sizeof(float4), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     E->obst_range_built = -1.0f;   // (re)bucketed at the next step
     s->envs_dirty = true;
@@ -1309,7 +1312,7 @@ static int upload_envs(ecm_sim* s) {
             EnvDesc& d = h[i];
             std::memset(&d, 0, sizeof(d));
             d.ag = E.ag; d.cell_base = E.cell_base;
-            d.n_obst_edges = E.n_obst_edges; d.oe0 = E.oe0.p; d.oe1 = E.oe1.p; d.oflags = E.oflags.p; d.og = E.og;
+            d.n_obst_edges = E.n_obst_edges; d.oe0 = E.oe0.p; d.oe1 = E.oe1.p; d.oe2 = E.oe2.p; d.og = E.og;
             d.obucket_start = E.obucket_start.p; d.obucket_edges = E.obucket_edges.p;
             d.n_cells = E.n_cells; d.cellA = E.cellA.p; d.cellB = E.cellB.p; d.eg = E.eg;
             d.ebucket_start = E.ebucket_start.p; d.ebucket_cells = E.ebucket_cells.p;
@@ -1565,7 +1568,7 @@ static int prepare_step(ecm_sim* s, DevState* out) {
 
 // 16 lanes per agent (row_kernels.h) for the plain step of a small crowd in
 // the default launch shape; other shapes say how agents are laid out.
-static constexpr int kRowAgents = 40000, kRowAttrAgents = 16000;
+static constexpr int kRowAgents = 160000, kRowAttrAgents = 16000;
 
 static void row_rule(ecm_sim* s, int mode) {
     // a crowd near a limit keeps the form it has: changing it captures the

@@ -31,8 +31,8 @@ struct EnvDesc {
     // obstacles (Environment::GetObstacles, edge per vertex in scan order)
     int n_obst_edges;
     const float4* oe0;      // (L.x, L.y, R.x, R.y),  R = next(L)
-    const float4* oe1;      // (prev(L).x, prev(L).y, next(R).x, next(R).y)
-    const uint8_t* oflags;  // bit0 convex(L), bit1 convex(R)
+    const float4* oe1;      // unit(L - prev(L)), unit(next(R) - R)
+    const float4* oe2;      // unit(R - L), |R - L|^2, flags: bit0 convex(L), bit1 convex(R)
     GridDesc og;
     const int* obucket_start;   // [side^2 + 1]
     const int* obucket_edges;   // ascending edge ids

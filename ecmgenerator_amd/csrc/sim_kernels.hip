@@ -1033,23 +1033,25 @@ __device__ __forceinline__ float4* q3d_slot(const DevState& s, uint32_t q, int c
 // Constraint::Contains, methodB (ORCA.h:49-60)
 __device__ __forceinline__ bool con_contains(const Con& c, V2 q) { return det(right(c.n), c.p - q) <= 0.0f; }
 
-// Obstacle half-plane for an edge (its oe0, oe1 and oflags; ORCA.cpp:70-333).
+// Obstacle half-plane for an edge (its oe0, oe1 and oe2; ORCA.cpp:70-333).
 // Returns false when the reference emits nothing for it (`continue` without
-// push_back).
-__device__ bool edge_constraint(const DevState& s, float4 a, float4 b, uint8_t fl, V2 position, V2 velocity, float rad,
-                                V2& outP, V2& outN) {
+// push_back).  The edge's direction and length and its neighbours' directions
+// do not depend on the agent: they are normalised once, on the host, which
+// takes 3 of the 5 roots and 6 of the 14 quotients out of every call.
+__device__ __forceinline__ bool edge_constraint(const DevState& s, float4 a, const float4& b, const float4& c,
+                                                V2 position, V2 velocity, float rad, V2& outP, V2& outN) {
     V2 pL = mk(a.x, a.y), pR = mk(a.z, a.w);
-    V2 pPrevL = mk(b.x, b.y), pNextR = mk(b.z, b.w);
+    const int fl = __float_as_int(c.w);
     bool cvL = fl & 1, cvR = (fl >> 1) & 1;
 
     V2 rp1 = pL - position;
     V2 rp2 = pR - position;
     V2 seg = pR - pL;
-    const float sp = dot(neg(rp1), seg) / len2(seg);
+    const float sp = dot(neg(rp1), seg) / c.z;
     const float distSqLine = len2(neg(rp1) - seg * sp);
     const float distSq1 = len2(rp1);
     const float distSq2 = len2(rp2);
-    seg = normalize(seg);
+    seg = mk(c.x, c.y);
     const float radiusSq = rad * rad;
 
     if (sp < 0.0f && distSq1 <= radiusSq) {                         // case 1
@@ -1057,8 +1059,7 @@ __device__ bool edge_constraint(const DevState& s, float4 a, float4 b, uint8_t f
         outP = mk(0.0f, 0.0f); outN = normalized(neg(rp1));
         return true;
     } else if (sp > 1.0f && distSq2 <= radiusSq) {                  // case 2
-        V2 rnd = normalize(pNextR - pR);
-        if (cvR && det(rp2, rnd) >= 0.0f) {
+        if (cvR && det(rp2, mk(b.z, b.w)) >= 0.0f) {
             outP = mk(0.0f, 0.0f); outN = normalized(neg(rp2));
             return true;
         }
@@ -1070,20 +1071,22 @@ __device__ bool edge_constraint(const DevState& s, float4 a, float4 b, uint8_t f
 
     // The obstacle's (L, R) pair, possibly collapsed to one vertex.  With
     // R := L, next(R) is the original R; with L := R, prev(L) is the
-    // original L.
-    V2 L = pL, R = pR, prevL = pPrevL, nextR = pNextR;
+    // original L: the direction to the neighbour is then the edge's own.
+    V2 L = pL, R = pR;
+    asm volatile("" ::: "memory");                  // b is read here, not held from the start
+    V2 lnd = mk(b.x, b.y), rnd = mk(b.z, b.w);      // unit(L - prev(L)), unit(next(R) - R)
     bool cL = cvL, cR = cvR;
     bool same = false;          // obstNeighborL == obstNeighborR (pointer identity)
     V2 leftLeg, rightLeg;
     if (sp < 0.0f && distSqLine <= radiusSq) {
         if (!cvL) return false;
-        R = pL; nextR = pR; cR = cvL; same = true;
+        R = pL; rnd = seg; cR = cvL; same = true;
         const float leg1 = sqrtf(distSq1 - radiusSq);
         leftLeg = mk(rp1.x * leg1 - rp1.y * rad, rp1.x * rad + rp1.y * leg1) / distSq1;
         rightLeg = mk(rp1.x * leg1 + rp1.y * rad, -rp1.x * rad + rp1.y * leg1) / distSq1;
     } else if (sp > 1.0f && distSqLine <= radiusSq) {
         if (!cvR) return false;
-        L = pR; prevL = pL; cL = cvR; same = true;
+        L = pR; lnd = seg; cL = cvR; same = true;
         const float leg2 = sqrtf(distSq2 - radiusSq);
         leftLeg = mk(rp2.x * leg2 - rp2.y * rad, rp2.x * rad + rp2.y * leg2) / distSq2;
         rightLeg = mk(rp2.x * leg2 + rp2.y * rad, -rp2.x * rad + rp2.y * leg2) / distSq2;
@@ -1103,9 +1106,7 @@ __device__ bool edge_constraint(const DevState& s, float4 a, float4 b, uint8_t f
     }
 
     bool leftForeign = false, rightForeign = false;
-    V2 lnd = normalize(L - prevL);
     if (cL && det(leftLeg, neg(lnd)) >= 0.0f) { leftLeg = neg(lnd); leftForeign = true; }
-    V2 rnd = normalize(nextR - R);
     if (cR && det(rightLeg, rnd) <= 0.0f) { rightLeg = rnd; rightForeign = true; }
 
     const float invT = s.inv_time_horizon_obst;
@@ -1148,7 +1149,7 @@ __device__ bool edge_constraint(const DevState& s, float4 a, float4 b, uint8_t f
 
 __device__ __forceinline__ bool obstacle_constraint(const DevState& s, const EnvDesc& E, int e, V2 position, V2 velocity,
                                                     float rad, V2& outP, V2& outN) {
-    return edge_constraint(s, E.oe0[e], E.oe1[e], E.oflags[e], position, velocity, rad, outP, outN);
+    return edge_constraint(s, E.oe0[e], E.oe1[e], E.oe2[e], position, velocity, rad, outP, outN);
 }
 
 // Agent half-plane (ORCA.cpp:339-423)
@@ -2254,7 +2255,7 @@ static void launch_orca_k(const DevState& s, int maxo, int mode, int oslots, int
 // rest of the plain step.  A wavefront for every four of `agents` (the kernel
 // strides, so that any count is covered).
 hipError_t launch_row_step(const DevState& s, int maxo, int agents, hipStream_t st) {
-    const int row_f4 = std::max(maxo, kRowLdsBytes / 16);
+    const int row_f4 = std::max(maxo + kRow, kRowLdsBytes / 16);
     hipLaunchKernelGGL(k_row_step, dim3(round8(cdiv(std::max(1, std::min(agents, s.n_slots)), 4))), dim3(64),
                        (size_t)row_f4 * 4 * sizeof(float4), st, s, maxo, row_f4);
     return hipGetLastError();
