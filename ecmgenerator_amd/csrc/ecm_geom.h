@@ -250,14 +250,13 @@ __device__ __forceinline__ float recip_from(float l, float y) {
     return __builtin_fmaf(__builtin_fmaf(-l, y, 1.0f), y, y);
 }
 // n / l for l > 0 and y its correctly rounded reciprocal, both in [2^-60,
-// 2^60), n zero or in [2^-80, 2^60) in magnitude; -0 / l gives +0
+// 2^60), n zero or in [2^-80, 2^60) in magnitude.  The residual is taken
+// negated: for n = -0 it is then +0, and the quotient -0.
 __device__ __forceinline__ float quot(float n, float l, float y) {
     const float q = n * y;
-    return __builtin_fmaf(__builtin_fmaf(-l, q, n), y, q);
+    return __builtin_fmaf(-__builtin_fmaf(l, q, -n), y, q);
 }
-__device__ __forceinline__ V2 quot(V2 n, float l, float y) {
-    return mk(__builtin_copysignf(quot(n.x, l, y), n.x), __builtin_copysignf(quot(n.y, l, y), n.y));
-}
+__device__ __forceinline__ V2 quot(V2 n, float l, float y) { return mk(quot(n.x, l, y), quot(n.y, l, y)); }
 // atan_f(x) for x in [0, 1]
 __device__ __forceinline__ float atan_unit(float x) {
     const bool red = x > 0.267949194f;

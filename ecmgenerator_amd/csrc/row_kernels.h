@@ -606,9 +606,10 @@ __device__ __forceinline__ void row_step_agent(const DevState& s, int t, int l, 
     if (fail < n) row_lp3d(C, an, ap, maxSpeed, fail, l, o);
     // the counters of the one-lane passes: 3D LPs, agents past the main
     // pass's obstacle slots, and both
-    wave_count(&s.stats[0], l == 0 && fail < n);
-    wave_count(&s.stats[1], l == 0 && C.nO > kRowStatObst);
-    wave_count(&s.stats[4], l == 0 && fail < n && C.nO > kRowStatObst);
+    uint32_t* ws = s.wstats + kStatStride * (blockIdx.x % kStatSlots);
+    wave_count(ws + kStat3d, l == 0 && fail < n);
+    wave_count(ws + kStatOvf, l == 0 && C.nO > kRowStatObst);
+    wave_count(ws + kStatBig, l == 0 && fail < n && C.nO > kRowStatObst);
     if (l == 0) integrate(s, t, position, velocity, o);
     row_fence();                                     // lds is reused by the next agent
 }

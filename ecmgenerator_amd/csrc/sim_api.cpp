@@ -98,6 +98,9 @@ static GridDesc make_grid(float x0, float y0, float x1, float y1, float cell, in
 // (kMaxBucketEdges + k constraints of 16 B per agent slot at most).
 constexpr int kMaxBucketEdges = 512;
 
+// words of the spread counters and the blocks' group counters behind them
+constexpr size_t kStatWords = (size_t)(kStatSlots + kDoneGroups) * kStatStride;
+
 struct EnvHost {
     float x0 = 0, y0 = 0, x1 = 0, y1 = 0;       // world box
     // obstacles
@@ -191,7 +194,7 @@ struct ecm_sim {
     // the 64-bit totals of finished steps live apart.
     static constexpr int kEventPeek = 1024;      // events read back while k_orca runs
     DBuf<uint32_t> xfer;                     // 8 + 4 * max_agents words
-    DBuf<uint32_t> wstats;                   // [64][4]
+    DBuf<uint32_t> wstats;                   // spread counters, then group_done
     DBuf<unsigned long long> acc;            // [16] totals (folded in by k_grid_count); [12] steps run
     // host-mapped, 1 + 8 + 4 * kEventPeek words: [0] the number of the last
     // step that published, then its counters and first events (written by
@@ -451,7 +454,7 @@ extern "C" int ecm_sim_create(const ecm_sim_params* p, float x0, float y0, float
     if (!rc) rc |= s->dead_ids.alloc(N);
     if (!rc) s->h_pending.assign(N, 0);
     if (!rc) rc |= s->xfer.alloc(8 + 4 * N);
-    if (!rc) rc |= s->wstats.alloc(256);
+    if (!rc) rc |= s->wstats.alloc(kStatWords);
     if (!rc) rc |= s->acc.alloc(16);
     if (!rc) rc |= s->agent_env.alloc(N);
     if (!rc && hipHostMalloc((void**)&s->h_xfer, (1 + 8 + 4 * (size_t)ecm_sim::kEventPeek) * sizeof(uint32_t),
@@ -485,7 +488,7 @@ extern "C" int ecm_sim_create(const ecm_sim_params* p, float x0, float y0, float
         rc |= zero_dev(s->radius.p, N * sizeof(float), s->stream);
         rc |= zero_dev(s->pref_speed.p, N * sizeof(float), s->stream);
         rc |= zero_dev(s->xfer.p, 8 * sizeof(uint32_t), s->stream);
-        rc |= zero_dev(s->wstats.p, 256 * sizeof(uint32_t), s->stream);
+        rc |= zero_dev(s->wstats.p, kStatWords * sizeof(uint32_t), s->stream);
         rc |= zero_dev(s->acc.p, 16 * sizeof(unsigned long long), s->stream);
         if (s->v_orca.p) rc |= zero_dev(s->v_orca.p, N * sizeof(float2), s->stream);
         if (!rc && hipStreamSynchronize(s->stream) != hipSuccess) rc = fail(ECM_E_HIP, "sync failed");
@@ -1367,6 +1370,7 @@ static DevState make_state(ecm_sim* s) {
     d.events = reinterpret_cast<int4*>(s->xfer.p + 8); d.events_n = s->xfer.p;
     d.stats = s->xfer.p + 2;
     d.wstats = s->wstats.p;
+    d.group_done = s->wstats.p + kStatSlots * kStatStride;
     d.acc = s->acc.p;
     d.host_xfer = s->h_xfer_dev;
     d.event_peek = (uint32_t)std::min(ecm_sim::kEventPeek, s->prm.max_agents);
@@ -1386,6 +1390,8 @@ static DevState make_state(ecm_sim* s) {
     d.q3d_agent = s->q3d_agent.p; d.q3d_info = s->q3d_info.p; d.q3d_vel = s->q3d_vel.p;
     d.q3d_con = s->q3d_con.p; d.con_stride = s->q3d_stride;
     d.q3d_cap = (uint32_t)s->prm.max_agents; d.q3d_big = s->q3d_big.p;
+    for (d.q3d_shift = 6; ((uint32_t)s->prm.max_agents + (1u << d.q3d_shift) - 1u) >> d.q3d_shift > kStatSlots;)
+        ++d.q3d_shift;
     d.k = s->prm.k;
     d.time_horizon = s->prm.time_horizon;
     {
@@ -2091,18 +2097,20 @@ extern "C" int ecm_sim_stats(ecm_sim* s, uint64_t* out, int n) {
     // device totals of the finished steps + the counters of the last step,
     // which the next step's grid build has not folded in yet
     unsigned long long acc[12];
-    uint32_t cur[8], ws[256];
+    uint32_t cur[8];
+    std::vector<uint32_t> ws((size_t)kStatSlots * kStatStride);
     HIPCHK(hipMemcpy(acc, s->acc.p, sizeof(acc), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(cur, s->xfer.p, sizeof(cur), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(ws, s->wstats.p, sizeof(ws), hipMemcpyDeviceToHost));
-    uint64_t col[4] = {acc[8], acc[9], acc[10], acc[11]};
-    for (int i = 0; i < 256; ++i) col[i & 3] += ws[i];
+    HIPCHK(hipMemcpy(ws.data(), s->wstats.p, ws.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    uint64_t col[kStatCols] = {acc[8], acc[9], acc[10]};
+    for (int i = 0; i < kStatSlots; ++i)
+        for (int c = 0; c < kStatCols; ++c) col[c] += ws[(size_t)i * kStatStride + c];
     uint64_t st[ECM_SIM_N_STATS];
     for (int i = 0; i < ECM_SIM_N_STATS; ++i) st[i] = s->stat[i];
-    st[2] = acc[2] + cur[2];        // 3D-LP queue
+    st[2] = acc[2] + col[kStat3d];          // agents whose 2D LP failed
     st[3] = acc[4] + cur[4];        // locate fallbacks
-    st[6] = acc[3] + cur[3];        // obstacle overflow queue
-    st[10] = acc[6] + cur[6];       // 3D-LP entries solved from the LDS tile
+    st[6] = acc[3] + cur[3] + col[kStatOvf];    // obstacle overflow queue
+    st[10] = acc[6] + cur[6] + col[kStatBig];   // 3D-LP entries solved from the LDS tile
     st[7] = col[0];
     st[8] = col[1];
     st[9] = col[2];

@@ -7,6 +7,18 @@
 
 namespace ecm {
 
+// Counters that every wavefront may add to are spread over kStatSlots slots of
+// kStatCols words, each slot on a line of its own (kStatStride words): atomics
+// on one address, or one line, take their turns at 20-30 ns each.
+constexpr int kStatSlots = 64, kStatStride = 64, kStatCols = 6;
+// columns: 0 learned proposals tried, 1 accepted, 2 constraints proposed, then
+constexpr int kStat3d = 3;      // agents whose 2D LP failed: the length of the 3D-LP queue's segment, or in
+                                // the row step counted by workgroup
+constexpr int kStatOvf = 4;     // row step: agents past the main pass's obstacle slots
+constexpr int kStatBig = 5;     // row step: both
+// First-level counters of the blocks that finished (publish_if_last).
+constexpr uint32_t kDoneGroups = 32;
+
 // Cell counts that one block of the grid build's prefix sum covers.
 constexpr uint32_t kScanCells = 4096;
 
@@ -130,12 +142,12 @@ struct DevState {
     // (id, x bits, y bits, 0) asks UpdatePath from the step-start position
     // (x, y); (id, 0, 0, 1) is a DestroyAgent.
     int4* events;         uint32_t* events_n;
-    uint32_t* stats;      // per step: [0] 3D-LP queue length, [1] obstacle-overflow queue
+    uint32_t* stats;      // per step: [0] unused, [1] obstacle-overflow queue
                           // length, [2] locate fallbacks to the exact-y list, [3] blocks of
                           // k_attr done, [4] 3D-LP entries with more obstacle constraints
                           // than the register tile holds, [5] unused
-    uint32_t* wstats;     // per step, [64][4] slots: learned proposals tried, accepted,
-                          // constraints proposed, unused
+    uint32_t* wstats;     // per step: the spread counters, [kStatSlots][kStatStride]
+    uint32_t* group_done; // [kDoneGroups][kStatStride] blocks of the attraction pass finished, by group
     unsigned long long* acc;   // [16] totals of the finished steps; [12] steps started,
                                // [13] the last grid's active count, [14] the previous one
     // host-mapped [1 + 8 + 4 * event_peek] words: [0] number of the last
@@ -152,6 +164,7 @@ struct DevState {
                             // at c * q3d_cap + q (q3d_slot)
     int con_stride;         // constraints per entry: MAXO + k
     uint32_t q3d_cap;       // entries the queue holds (max_agents)
+    uint32_t q3d_shift;     // segments of 2^q3d_shift entries, at most kStatSlots of them
     int* q3d_big;           // entries with more obstacle constraints than the register tile
 
     // ---- learned proposal ----

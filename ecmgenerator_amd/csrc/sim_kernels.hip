@@ -70,23 +70,33 @@ __device__ __forceinline__ int xcd_block() {
 
 // ------------------------------------------------------------ grid build
 // Start of a step (block 0 of k_grid_count, 256 threads): add the
-// previous step's counters (8 words) and the column sums of the
-// per-wavefront slots ([64][4] words) to the 64-bit totals (acc[0..7] and
-// acc[8..11]), count the step (acc[12]), then clear both for this step.
+// previous step's counters (8 words) and the column sums of the spread ones
+// to the 64-bit totals (acc[0..7], with the last three columns among them,
+// and acc[8..10]), count the step (acc[12]), then clear both for this step.
 // No other block of the grid touches them.
 __device__ __forceinline__ void step_begin(uint32_t* counters, uint32_t* wstats, unsigned long long* acc) {
-    __shared__ uint32_t col[4];
+    __shared__ uint32_t col[kStatCols];
     const int t = threadIdx.x;
-    if (t < 4) col[t] = 0u;
+    if (t < kStatCols) col[t] = 0u;
     __syncthreads();
-    const uint32_t w = wstats[t];
-    if (w) atomicAdd(&col[t & 3], w);
+    for (int i = t; i < kStatSlots * kStatCols; i += 256) {
+        uint32_t* at = wstats + (i % kStatSlots) * kStatStride + i / kStatSlots;
+        const uint32_t w = *at;
+        if (w) {
+            atomicAdd(&col[i / kStatSlots], w);
+            *at = 0u;
+        }
+    }
     const uint32_t c = t < 8 ? counters[t] : 0u;
     __syncthreads();
-    if (t < 8) { acc[t] += c; counters[t] = 0u; }
-    if (t < 4) acc[8 + t] += col[t];
+    if (t < 8) {
+        // counters and totals [2], [3] and [6] are stats[0], [1] and [4]
+        const uint32_t more = t == 2 ? col[kStat3d] : t == 3 ? col[kStatOvf] : t == 6 ? col[kStatBig] : 0u;
+        acc[t] += (unsigned long long)c + more;
+        counters[t] = 0u;
+    }
+    if (t < 3) acc[8 + t] += col[t];
     if (t == 0) acc[12] += 1ull;
-    wstats[t] = 0u;
 }
 
 // Histogram pass, entered from the slot-indexed arrays: one element per
@@ -908,7 +918,20 @@ __device__ __forceinline__ void knn_agent(const DevState& s, int* knn_lds, int t
 __device__ __forceinline__ void publish_if_last(const DevState& s) {
     __shared__ uint32_t last;
     __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(s.blocks_done, 1u) == gridDim.x - 1u ? 1u : 0u;
+    if (threadIdx.x == 0) {
+        // through kDoneGroups counters first: one address takes an atomic
+        // each 20-30 ns, and a million agents have 3,700 blocks
+        bool l = true;
+        uint32_t n = gridDim.x;
+        if (n > 2 * kDoneGroups) {
+            const uint32_t g = blockIdx.x % kDoneGroups;
+            uint32_t* at = s.group_done + g * kStatStride;
+            l = atomicAdd(at, 1u) == (n - g + kDoneGroups - 1) / kDoneGroups - 1u;
+            if (l) *at = 0u;
+            n = kDoneGroups;
+        }
+        last = l && atomicAdd(s.blocks_done, 1u) == n - 1u ? 1u : 0u;
+    }
     __syncthreads();
     if (!last) return;
     __threadfence();
@@ -1464,6 +1487,18 @@ __device__ __forceinline__ uint32_t wave_alloc(uint32_t* ctr) {
     return base + (uint32_t)__popcll(act & ((1ull << lane) - 1ull));
 }
 
+// An entry of the 3D-LP queue for each active lane, in the segment of its
+// agent (sorted position t): 64 segments at most, each with a counter on a
+// line of its own and as many entries as agents, so none overflows.
+__device__ __forceinline__ uint32_t queue_alloc(const DevState& s, int t) {
+    const uint32_t seg = (uint32_t)t >> s.q3d_shift;
+    const uint32_t first = __builtin_amdgcn_readfirstlane(seg);
+    uint32_t at;
+    if (__ballot(seg != first) == 0ull) at = wave_alloc(s.wstats + first * kStatStride + kStat3d);
+    else at = atomicAdd(s.wstats + seg * kStatStride + kStat3d, 1u);
+    return (seg << s.q3d_shift) + at;
+}
+
 // Count `pred` over the active lanes of the wavefront with one atomic.
 __device__ __forceinline__ void wave_count(uint32_t* ctr, bool pred) {
     const unsigned long long b = __ballot(pred);
@@ -1602,6 +1637,7 @@ __device__ __forceinline__ void orca_agent(const DevState& s, int t, float4* lds
     }
     {
         // all neighbour loads issued before the first constraint
+        uint32_t redo = 0u;
         float4 q[K];
         float2 qv[K];
 #pragma unroll
@@ -1614,10 +1650,18 @@ __device__ __forceinline__ void orca_agent(const DevState& s, int t, float4* lds
         for (int j = 0; j < K; ++j) {
             if (j < cnt) {
                 V2 cp, cn;
-                agent_constraint(s, position, velocity, rad, q[j], qv[j], cp, cn);
+                if (s.inv_dt == 0.0f) agent_constraint(s, position, velocity, rad, q[j], qv[j], cp, cn);
+                else if (!agent_constraint_common(s, position, velocity, rad, q[j], qv[j], cp, cn)) redo |= 1u << j;
                 con_st(lds, TL, nc, cp, cn);
                 ++nc;
             }
+        }
+        for (; redo; redo &= redo - 1u) {
+            const int j = __ffs((int)redo) - 1;
+            const int sj = s.nbr[(size_t)j * s.n_slots + t];
+            V2 cp, cn;
+            agent_constraint(s, position, velocity, rad, s.sorted_pr[sj], sorted_vel(s, sj), cp, cn);
+            con_st(lds, TL, nObst + j, cp, cn);
         }
     }
 
@@ -1638,7 +1682,7 @@ __device__ __forceinline__ void orca_agent(const DevState& s, int t, float4* lds
             if (!((cm >> c) & 1u) && !con_contains(con_ld(lds, TL, c), o)) ok = false;
         // per-wavefront counters spread over 64 slots (one address each
         // would serialize 15k atomics per launch)
-        uint32_t* ws = s.wstats + 4 * (blockIdx.x & 63);
+        uint32_t* ws = s.wstats + kStatStride * (blockIdx.x % kStatSlots);
         wave_count(ws + 0, true);
         wave_count(ws + 1, ok);
         wave_sum5(ws + 2, (uint32_t)__popc(cm));
@@ -1653,7 +1697,7 @@ __device__ __forceinline__ void orca_agent(const DevState& s, int t, float4* lds
     if (fail < nc) {
         // RandomizedLP3D runs on a compacted queue: park the constraints,
         // the 2D result and the failing index
-        uint32_t q = wave_alloc(&s.stats[0]);
+        uint32_t q = queue_alloc(s, t);
         s.q3d_agent[q] = t;
         s.q3d_info[q] = make_int4(nc, nObst, fail, 0);
         s.q3d_vel[q] = make_float2(o.x, o.y);
@@ -1811,7 +1855,7 @@ __device__ __forceinline__ void orca_reg_agent(const DevState& s, int t) {
     }
     const int cnt = s.nbr_cnt[t];
     V2 an[K], ap[K];
-    uint32_t aval = 0u;
+    uint32_t aval = 0u, redo = 0u;
     // the neighbours' loads in batches of kNbrBatch, each batch issued before
     // its constraints are built: the loads of a batch are in flight together,
     // and the batch's 6 registers per neighbour stay within the 80-VGPR cap
@@ -1836,17 +1880,29 @@ __device__ __forceinline__ void orca_reg_agent(const DevState& s, int t) {
                 an[j] = mk(0.0f, 0.0f);
                 ap[j] = mk(0.0f, 0.0f);
                 if (j < cnt) {
-                    agent_constraint(s, position, velocity, rad, q[u], qv[u], ap[j], an[j]);
+                    if (s.inv_dt == 0.0f) agent_constraint(s, position, velocity, rad, q[u], qv[u], ap[j], an[j]);
+                    else if (!agent_constraint_common(s, position, velocity, rad, q[u], qv[u], ap[j], an[j]))
+                        redo |= 1u << j;
                     aval |= 1u << j;
                 }
             }
         }
     }
+    // the few whose operands the cheap form does not cover
+    for (; redo; redo &= redo - 1u) {
+        const int j = __ffs((int)redo) - 1;
+        const int sj = s.nbr[(size_t)j * s.n_slots + t];
+        V2 cp, cn;
+        agent_constraint(s, position, velocity, rad, s.sorted_pr[sj], sorted_vel(s, sj), cp, cn);
+#pragma unroll
+        for (int u = 0; u < K; ++u)
+            if (u == j) { ap[u] = cp; an[u] = cn; }
+    }
     V2 o;
     const int fs = lp2_reg<OB, K>(on, op, OB - nObst, an, ap, aval, mk(pv.x, pv.y), maxSpeed, o);
     if (fs < OB + K) {
         // RandomizedLP3D runs on the compacted queue (k_lp3d_reg)
-        const uint32_t qi = wave_alloc(&s.stats[0]);
+        const uint32_t qi = queue_alloc(s, t);
         s.q3d_agent[qi] = t;
         s.q3d_info[qi] = make_int4(nObst + cnt, nObst, slot_to_index<OB>(fs, nObst), 0);
         s.q3d_vel[qi] = make_float2(o.x, o.y);
@@ -1924,7 +1980,7 @@ __device__ __forceinline__ void orca_agent_wave(const DevState& s, int t, float4
         const int fail = lp2d(lds, T, nc, nc, 0, mk(pv.x, pv.y), maxSpeed, false, o);
         if (fail < nc) {
             // RandomizedLP3D runs on the compacted queue, as from orca_agent
-            const uint32_t qi = wave_alloc(&s.stats[0]);
+            const uint32_t qi = queue_alloc(s, t);
             s.q3d_agent[qi] = t;
             s.q3d_info[qi] = make_int4(nc, nObst, fail, 0);
             s.q3d_vel[qi] = make_float2(o.x, o.y);
@@ -2037,15 +2093,26 @@ static constexpr uint32_t kLp3dSpreadLanes = 4;
 // wave-uniform: a full wavefront runs the union of its lanes').
 template <int K, int OB>
 __global__ __launch_bounds__(256, 4) void k_lp3d_reg(DevState s) {
-    const uint32_t nq = s.stats[0];
     const uint32_t lane = threadIdx.x & 63u;
+    // the segments' lengths, one per lane, as one list
+    const uint32_t len_l = s.wstats[lane * kStatStride + kStat3d];
+    const uint32_t end_l = wave_incl_scan(len_l);
+    const uint32_t nq = __shfl(end_l, 63);
+    if (nq == 0u) return;
     const uint32_t wpb = blockDim.x >> 6;
     const uint32_t nw = gridDim.x * wpb;
     const uint32_t w0 = blockIdx.x + gridDim.x * (threadIdx.x >> 6);
     const bool spread = nq <= nw * kLp3dSpreadLanes;
     for (uint32_t w = w0; spread ? w == w0 : w * 64u < nq; w += nw) {
-        const uint32_t q = spread ? lane * nw + w : w * 64u + lane;
-        if (q >= nq) continue;
+        const uint32_t f = spread ? lane * nw + w : w * 64u + lane;
+        // its segment: the number of segments that end at or before f
+        const uint32_t fc = min(f, nq - 1u);
+        uint32_t seg = 0;
+#pragma unroll
+        for (uint32_t h = 32; h; h >>= 1)
+            if ((uint32_t)__shfl(end_l, (int)(seg + h - 1u)) <= fc) seg += h;
+        const uint32_t q = (seg << s.q3d_shift) + fc - (uint32_t)__shfl(end_l - len_l, (int)seg);
+        if (f >= nq) continue;
         const int4 info = s.q3d_info[q];
         const int nObst = info.y, na = info.x - info.y;
         if (nObst > OB) {
