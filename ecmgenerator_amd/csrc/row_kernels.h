@@ -62,18 +62,11 @@ __device__ __forceinline__ int row_locate_cell(const EnvDesc& s, V2 p, int l, ui
     const int bx = grid_cell(p.x, s.eg.x0, s.eg.inv_cell, s.eg.side);
     const int by = grid_cell(p.y, s.eg.y0, s.eg.inv_cell, s.eg.side);
     const int b = by * s.eg.side + bx;
+    const uint32_t key = (p.y == 0.0f) ? 0u : __float_as_uint(p.y);
+    uint32_t h = hash_u32(key) & (uint32_t)s.yhash_mask;
+    uint32_t kk = 0xffffffffu;
+    if (s.yhash_mask >= 0) kk = s.yhash_key[h];
     const int i0 = s.ebucket_start[b], ie = s.ebucket_start[b + 1];
-    int j0 = 0, je = 0;
-    if (s.yhash_mask >= 0) {
-        const uint32_t key = (p.y == 0.0f) ? 0u : __float_as_uint(p.y);
-        uint32_t h = hash_u32(key) & (uint32_t)s.yhash_mask;
-        while (true) {
-            const uint32_t kk = s.yhash_key[h];
-            if (kk == 0xffffffffu) break;
-            if (kk == key) { j0 = s.yhash_off[h]; je = j0 + s.yhash_cnt[h]; fallback = 1; break; }
-            h = (h + 1u) & (uint32_t)s.yhash_mask;
-        }
-    }
     int best = INT_MAX;
     auto scan = [&](const int* list, int a, int e) {
         for (int i = a; i < e; i += kRow) {
@@ -92,14 +85,21 @@ __device__ __forceinline__ int row_locate_cell(const EnvDesc& s, V2 p, int l, ui
         }
     };
     scan(s.ebucket_cells, i0, ie);
-    scan(s.ycells, j0, je);
+    while (kk != 0xffffffffu) {
+        if (kk == key) {
+            const int j0 = s.yhash_off[h];
+            scan(s.ycells, j0, j0 + s.yhash_cnt[h]);
+            fallback = 1;
+            break;
+        }
+        h = (h + 1u) & (uint32_t)s.yhash_mask;
+        kk = s.yhash_key[h];
+    }
     return best == INT_MAX ? -1 : best;
 }
 
 // irm_attraction with one path segment per lane, 16 from the end at a time.
-__device__ __forceinline__ bool row_irm(const EnvDesc& s, V2 pos, const float2* path, int np, int l, V2& out,
-                                        uint32_t& fb) {
-    const int cell = row_locate_cell(s, pos, l, fb);
+__device__ __forceinline__ bool row_irm(const EnvDesc& s, V2 pos, int cell, const float2* path, int np, int l, V2& out) {
     if (cell < 0) return false;
     V2 rl = mk(0.0f, 0.0f), oa, ob;
     if (!retract(s, pos, cell, rl, oa, ob)) return false;
@@ -157,25 +157,24 @@ __device__ __forceinline__ void row_attr_agent(const DevState& s, int t, int l, 
     const int np = in.pc.y;
     const float2* path = s.path_pts + in.pc.x;
     const float2 gg = path[np - 1];
+    uint32_t fb = 0;
+    const int cell = row_locate_cell(E, pos, l, fb);
     const float gx = pos.x - gg.x, gy = pos.y - gg.y;
     const float dGoal = gx * gx + gy * gy;
     V2 attr = mk(in.a0.x, in.a0.y);
     bool alive = true, event = false;
-    uint32_t fb = 0;
     if (dGoal < s.arrival_r2) {
         attr = mk(gg.x, gg.y);
         if (dGoal < s.delete_r2) alive = false;
+        fb = 0;
     } else {
         V2 ap = mk(0.0f, 0.0f);
-        if (row_irm(E, pos, path, np, l, ap, fb)) attr = ap;
+        if (row_irm(E, pos, cell, path, np, l, ap)) attr = ap;
         else event = true;
     }
     if (l != 0) return;
-    if (event) {
-        // UpdatePath(e, currentPosition, goal) with the step-start position
-        const uint32_t q = atomicAdd(s.events_n, 1u);
-        s.events[q] = make_int4(__float_as_int(in.pr.w), __float_as_int(pos.x), __float_as_int(pos.y), t);
-    }
+    // UpdatePath(e, currentPosition, goal) with the step-start position
+    if (event) put_event(s, __float_as_int(in.pr.w), __float_as_int(pos.x), __float_as_int(pos.y), t);
     s.attr_s[t] = make_float2(attr.x, attr.y);
     if (fb) atomicAdd(&s.stats[2], 1u);
     s.dead_s[t] = alive ? 0 : 1;
@@ -185,7 +184,6 @@ __device__ __forceinline__ void row_attr_agent(const DevState& s, int t, int l, 
     }
     const V2 des = normalize(attr - pos) * in.sv.z;
     s.pref_vel_s[t] = make_float2(des.x, des.y);
-    if (event) __threadfence();
 }
 
 // k_attr and k_scatter_attr with 16 lanes per agent: 14 -> 10 us at 500 agents
@@ -196,21 +194,27 @@ __global__ __launch_bounds__(256) void k_attr_row(DevState s) {
     const int per = blockDim.x / kRow, l = threadIdx.x & (kRow - 1);
     for (int t = xcd_block() * per + (int)threadIdx.x / kRow; t < n_active; t += gridDim.x * per)
         row_attr_agent(s, t, l, attr_in(s, t));
-    publish_if_last(s);
+    publish_if_last(s, gridDim.x);
 }
 
-__global__ __launch_bounds__(256) void k_scatter_attr_row(DevState s) {
-    __shared__ uint32_t top[kTopMax];
-    const Starts S = scatter_starts(s, top);
+__global__ __launch_bounds__(256) void k_scatter_attr_row(DevState s, uint32_t blocks) {
+    __shared__ __align__(16) uint32_t top[kTopMax];
+    if (blockIdx.x >= blocks) { write_starts(s, blockIdx.x - blocks); return; }
     const int n_old = (int)(uint32_t)s.acc[14], n = n_old + (int)(uint32_t)s.acc[15];
     const int per = blockDim.x / kRow, l = threadIdx.x & (kRow - 1);
-    for (int t = xcd_block() * per + (int)threadIdx.x / kRow; t < n; t += gridDim.x * per) {
-        const uint32_t m = s.key[t];
-        if (m == kInvalidKey) continue;
-        const int slot = (int)(S.at(m) + s.rank[t]);
-        row_attr_agent(s, slot, l, scatter_agent(s, t, n_old, slot, l == 0));
+    int t = xcd_block((int)blocks) * per + (int)threadIdx.x / kRow;
+    Moved M = moved_agent(s, t, n_old, n);
+    const Starts S = scatter_starts(s, top);
+    while (t < n) {
+        if (M.m != kInvalidKey) {
+            const int slot = (int)(S.pre[M.m / kScanCells] + M.in_cell);
+            if (l == 0) store_moved(s, M.in, slot);
+            row_attr_agent(s, slot, l, M.in);
+        }
+        t += (int)blocks * per;
+        M = moved_agent(s, t, n_old, n);
     }
-    publish_if_last(s);
+    publish_if_last(s, blocks);
 }
 
 // ------------------------------------------------------------- neighbours

@@ -1290,10 +1290,12 @@ static int ensure_agent_grid(ecm_sim* s) {
     const size_t GP = (G + kScanCells - 1) / kScanCells * kScanCells;
     rc = s->cell_count.alloc(GP);
     if (!rc) rc = s->cell_local.alloc(GP);
-    if (!rc) rc = s->cell_start.alloc(G + 1);
-    if (!rc) rc = s->bsum.alloc(GP / kScanCells);
+    if (!rc) rc = s->cell_start.alloc(GP + 1);
+    const size_t nb = std::max(GP / kScanCells, (size_t)kScanTop);
+    if (!rc) rc = s->bsum.alloc(nb);
     if (rc) return rc;
     rc = zero_dev(s->cell_count.p, GP * sizeof(uint32_t), s->stream);
+    if (!rc) rc = zero_dev(s->bsum.p, nb * sizeof(uint32_t), s->stream);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(s->stream));
     s->n_keys = (uint32_t)G;
@@ -1625,8 +1627,8 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
     return 0;
 }
 
-// Waits until step `seq` has published its events (k_attr writes the
-// step number last, after a system-scope fence).  The stream is polled
+// Waits until step `seq` has published its events (the attraction pass stores
+// the step number last, when its other words have arrived).  The stream is polled
 // now and then so that a step that ends without publishing is an error,
 // not a hang.
 static int wait_published(ecm_sim* s, uint32_t seq) {

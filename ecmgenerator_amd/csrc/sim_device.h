@@ -21,6 +21,9 @@ constexpr uint32_t kDoneGroups = 32;
 
 // Cell counts that one block of the grid build's prefix sum covers.
 constexpr uint32_t kScanCells = 4096;
+// Block totals that a block of the scatter scans in LDS: bsum holds at least
+// as many, zeros past the grid's.
+constexpr uint32_t kScanTop = 2048;
 
 // Uniform grid over the world box.  Cell (cx, cy) of a point is
 // floor((p - origin) / cell), clamped to [0, side); NaN maps to 0.
@@ -122,7 +125,7 @@ struct DevState {
     uint32_t* cell_count;   // [n_keys, padded to scan blocks] zero between steps (the scan clears it)
     uint32_t* cell_local;   // [n_keys, padded as cell_count] exclusive scan within a scan block
     uint32_t* bsum;         // [scan blocks] agents per scan block
-    uint32_t* cell_start;   // [n_keys + 1] exclusive scan; [n_keys] = active count
+    uint32_t* cell_start;   // [n_keys, padded as cell_count, + 1] exclusive scan; [n_keys] = active count
     float4* sorted_pr;      // [n_slots] (x, y, radius, id bits)
     float4* sorted_v;       // [n_slots] (vx, vy, preferred speed, environment bits)
     int* nbr;               // [k][n_slots] neighbour sorted positions (SoA)

@@ -62,10 +62,19 @@ __device__ __forceinline__ uint32_t cell_key(const EnvDesc& E, float2 p) {
 
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup i -> XCD i % 8).
 // Remap so that XCD x processes the x-th contiguous eighth of the Morton
-// order: neighbouring agents then share one L2.  gridDim.x is a multiple of 8.
-__device__ __forceinline__ int xcd_block() {
-    const int per = gridDim.x >> 3;
+// order: neighbouring agents then share one L2.  `blocks`, a multiple of 8, of
+// the grid's workgroups (the first) work on agents.
+__device__ __forceinline__ int xcd_block(int blocks) {
+    const int per = blocks >> 3;
     return (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+}
+__device__ __forceinline__ int xcd_block() { return xcd_block((int)gridDim.x); }
+
+// Waits until this wavefront's stores are done, and keeps the compiler from
+// moving memory accesses across.
+__device__ __forceinline__ void stores_done() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // ------------------------------------------------------------ grid build
@@ -191,12 +200,15 @@ __device__ __forceinline__ uint32_t block_excl_scan256(uint32_t v, uint32_t& tot
 }
 // The prefix sum of the cell counts takes one launch and part of the scatter:
 // k_scan_local scans kScanCells counts per block into cell_local and the
-// block's total into bsum; every block of the scatter scans the totals again
-// in LDS (a few hundred: under a microsecond, behind its own loads), adds
-// them where it needs a cell's start and writes its share of cell_start.  As
-// a scan of the totals and an add pass of their own these were two launches
-// more, 4-5 us and a 1.5 us gap each whatever the crowd's size.
-static constexpr uint32_t kTopMax = 2048;        // block totals a scatter block scans in LDS
+// block's total into bsum; every block of the scatter that places agents scans
+// the totals again in LDS (a few hundred: under a microsecond, behind its own
+// loads) and adds them where it needs a cell's start, and further blocks of
+// the same launch, one per scan block, write cell_start.  As a scan of the
+// totals and an add pass of their own these were two launches more, 4-5 us and
+// a 1.5 us gap each whatever the crowd's size; with cell_start written by the
+// blocks that place agents, a crowd spread over many cells waited for it (28
+// dependent loads a thread for 37,000 agents on a million cells).
+static constexpr uint32_t kTopMax = kScanTop;
 // kScanCells counts per block; the counts are cleared for the next step.
 // Both arrays are padded to whole blocks.
 __global__ __launch_bounds__(256) void k_scan_local(uint4* cnt, uint4* local, uint32_t* bsum) {
@@ -251,28 +263,51 @@ struct Starts {
     const uint32_t* pre;
     __device__ __forceinline__ uint32_t at(uint32_t m) const { return local[m] + pre[m / kScanCells]; }
 };
-// The first part of every scatter kernel (256 threads, all of them).
+// The first part of every block that places agents (256 threads, all of them).
 __device__ __forceinline__ Starts scatter_starts(const DevState& s, uint32_t* top) {
     const uint32_t nb = (s.n_keys + kScanCells - 1) / kScanCells;
-    Starts S{s.cell_local, s.bsum};
-    if (nb <= kTopMax) {
-        uint32_t carry = 0;
-        for (uint32_t c = 0; c < nb; c += 256u) {
-            const uint32_t i = c + threadIdx.x;
-            uint32_t tot;
-            const uint32_t ex = block_excl_scan256(i < nb ? s.bsum[i] : 0u, tot);
-            if (i < nb) top[i] = carry + ex;
-            carry += tot;
-        }
-        __syncthreads();
-        S.pre = top;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            s.cell_start[s.n_keys] = carry;
-            s.acc[13] = carry;
-        }
+    if (nb > kTopMax) return Starts{s.cell_local, s.bsum};
+    // bsum is padded with zeros to kTopMax totals
+    uint32_t tot;
+    if (nb <= 256u) {
+        top[threadIdx.x] = block_excl_scan256(s.bsum[threadIdx.x], tot);
+    } else {
+        const uint4* b = reinterpret_cast<const uint4*>(s.bsum) + threadIdx.x * 2;
+        const uint4 u = b[0], v = b[1];
+        uint4 x, y;
+        x.x = block_excl_scan256(u.x + u.y + u.z + u.w + v.x + v.y + v.z + v.w, tot);
+        x.y = x.x + u.x; x.z = x.y + u.y; x.w = x.z + u.z;
+        y.x = x.w + u.w; y.y = y.x + v.x; y.z = y.y + v.y; y.w = y.z + v.z;
+        uint4* o = reinterpret_cast<uint4*>(top) + threadIdx.x * 2;
+        o[0] = x;
+        o[1] = y;
     }
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < s.n_keys; i += gridDim.x * 256u) s.cell_start[i] = S.at(i);
-    return S;
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        s.cell_start[s.n_keys] = tot;
+        s.acc[13] = tot;
+    }
+    return Starts{s.cell_local, top};
+}
+// Block e of the others: the starts of scan block e's cells.
+__device__ __forceinline__ void write_starts(const DevState& s, uint32_t e) {
+    const uint32_t nb = (s.n_keys + kScanCells - 1) / kScanCells;
+    const uint4* in = reinterpret_cast<const uint4*>(s.cell_local) + (size_t)e * (kScanCells / 4) + threadIdx.x;
+    uint4 c[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) c[q] = in[q * 256];
+    uint32_t pre = 0;
+    if (nb > kTopMax) {
+        pre = s.bsum[e];
+    } else {
+        uint32_t sum = 0;
+        for (uint32_t i = threadIdx.x; i < e; i += 256u) sum += s.bsum[i];
+        block_excl_scan256(sum, pre);
+    }
+    uint4* out = reinterpret_cast<uint4*>(s.cell_start) + (size_t)e * (kScanCells / 4) + threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        out[q * 256] = make_uint4(c[q].x + pre, c[q].y + pre, c[q].z + pre, c[q].w + pre);
 }
 
 // Counting-sort scatter from the slot-indexed arrays: the sorted position
@@ -282,8 +317,9 @@ __device__ __forceinline__ Starts scatter_starts(const DevState& s, uint32_t* to
 // there) keeps its neighbour seeds: prev_of and fwd link u and its new
 // position.  Any k distinct agents bound the k-th distance, so seeds stay
 // safe after spawns, removals, writes and loads.
-__global__ __launch_bounds__(256) void k_grid_scatter(DevState s) {
-    __shared__ uint32_t top[kTopMax];
+__global__ __launch_bounds__(256) void k_grid_scatter(DevState s, uint32_t blocks) {
+    __shared__ __align__(16) uint32_t top[kTopMax];
+    if (blockIdx.x >= blocks) { write_starts(s, blockIdx.x - blocks); return; }
     const Starts S = scatter_starts(s, top);
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= s.n_slots) return;
@@ -339,34 +375,49 @@ __device__ __forceinline__ uint32_t hash_u32(uint32_t x) {
 // linear scan of ECMCellCollection::PointLocationQueryLinear: a cell can only
 // contain p if p lies in its (margin-expanded) box, except when p.y equals
 // the y of one of its vertices exactly; those cells are listed per y value.
-__device__ int locate_cell(const EnvDesc& s, V2 p, uint32_t& fallback) {
+// Both lists ascend: the first is the lower of their first hits.  Four list
+// entries, and two rings, are loaded together: a wavefront waits out its
+// longest list, and one entry at a time it waited for two loads an entry.
+__device__ __forceinline__ int locate_cell(const EnvDesc& s, V2 p, uint32_t& fallback) {
     if (s.n_cells == 0) return -1;
     int bx = grid_cell(p.x, s.eg.x0, s.eg.inv_cell, s.eg.side);
     int by = grid_cell(p.y, s.eg.y0, s.eg.inv_cell, s.eg.side);
     int b = by * s.eg.side + bx;
-    int i = s.ebucket_start[b], ie = s.ebucket_start[b + 1];
-    int j = 0, je = 0;
-    if (s.yhash_mask >= 0) {
-        uint32_t key = (p.y == 0.0f) ? 0u : __float_as_uint(p.y);
-        uint32_t h = hash_u32(key) & (uint32_t)s.yhash_mask;
-        while (true) {
-            uint32_t kk = s.yhash_key[h];
-            if (kk == 0xffffffffu) break;
-            if (kk == key) { j = s.yhash_off[h]; je = j + s.yhash_cnt[h]; fallback = 1; break; }
-            h = (h + 1u) & (uint32_t)s.yhash_mask;
+    const uint32_t key = (p.y == 0.0f) ? 0u : __float_as_uint(p.y);
+    uint32_t h = hash_u32(key) & (uint32_t)s.yhash_mask;
+    uint32_t kk = 0xffffffffu;
+    if (s.yhash_mask >= 0) kk = s.yhash_key[h];
+    const int i0 = s.ebucket_start[b], ie = s.ebucket_start[b + 1];
+    int best = INT_MAX;
+    for (int i = i0; i < ie && best == INT_MAX; i += 4) {
+        int c[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c[u] = s.ebucket_cells[min(i + u, ie - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u += 2) {
+            if (i + u < ie && best == INT_MAX) {
+                const float4 A = s.cellA[c[u]], B = s.cellB[c[u]], C = s.cellA[c[u + 1]], D = s.cellB[c[u + 1]];
+                if (quad_contains(p, mk(A.x, A.y), mk(A.z, A.w), mk(B.x, B.y), mk(B.z, B.w))) best = c[u];
+                else if (quad_contains(p, mk(C.x, C.y), mk(C.z, C.w), mk(D.x, D.y), mk(D.z, D.w))) best = c[u + 1];
+            }
         }
     }
-    while (i < ie || j < je) {
-        int ci = i < ie ? s.ebucket_cells[i] : INT_MAX;
-        int cj = j < je ? s.ycells[j] : INT_MAX;
-        int c;
-        if (ci < cj) { c = ci; ++i; }
-        else if (cj < ci) { c = cj; ++j; }
-        else { c = ci; ++i; ++j; }
-        float4 A = s.cellA[c], B = s.cellB[c];
-        if (quad_contains(p, mk(A.x, A.y), mk(A.z, A.w), mk(B.x, B.y), mk(B.z, B.w))) return c;
+    while (kk != 0xffffffffu) {
+        if (kk == key) {
+            fallback = 1;
+            const int j0 = s.yhash_off[h], je = j0 + s.yhash_cnt[h];
+            for (int j = j0; j < je; ++j) {
+                const int c = s.ycells[j];
+                if (c >= best) break;
+                const float4 A = s.cellA[c], B = s.cellB[c];
+                if (quad_contains(p, mk(A.x, A.y), mk(A.z, A.w), mk(B.x, B.y), mk(B.z, B.w))) { best = c; break; }
+            }
+            break;
+        }
+        h = (h + 1u) & (uint32_t)s.yhash_mask;
+        kk = s.yhash_key[h];
     }
-    return -1;
+    return best == INT_MAX ? -1 : best;
 }
 
 // ECM::RetractPoint (ECM.cpp:20-96) given the located cell.  Cell 2e holds
@@ -394,8 +445,7 @@ __device__ bool retract(const EnvDesc& s, V2 loc, int cell, V2& out, V2& oa, V2&
 }
 
 // IRMPathFollower::FindAttractionPoint (IRMPathFollower.cpp:14-115)
-__device__ bool irm_attraction(const EnvDesc& s, V2 pos, const float2* path, int np, V2& out, uint32_t& fb) {
-    int cell = locate_cell(s, pos, fb);
+__device__ __forceinline__ bool irm_attraction(const EnvDesc& s, V2 pos, int cell, const float2* path, int np, V2& out) {
     if (cell < 0) return false;
     V2 rl = mk(0.0f, 0.0f), oa, ob;
     if (!retract(s, pos, cell, rl, oa, ob)) return false;
@@ -814,10 +864,23 @@ __device__ __forceinline__ AttrIn attr_in(const DevState& s, int t) {
     return AttrIn{s.sorted_pr[t], s.sorted_v[t], s.path_s[t], s.attr_s[t], s.prev_of[t]};
 }
 
+// Appends an event.  The last block of the launch reads it (publish_if_last),
+// perhaps on another XCD: stored past the L2 and waited for, before the
+// block counts itself as done.  A device fence instead writes back whatever
+// the XCD's L2 holds, some 8 us and a hundred times a step at a million agents.
+__device__ __forceinline__ void put_event(const DevState& s, int x, int y, int z, int w) {
+    const uint32_t q = atomicAdd(s.events_n, 1u);
+    unsigned long long* at = reinterpret_cast<unsigned long long*>(s.events + q);
+    auto two = [](int lo, int hi) { return (unsigned long long)(uint32_t)lo | (unsigned long long)(uint32_t)hi << 32; };
+    __hip_atomic_store(at, two(x, y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(at + 1, two(z, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    stores_done();
+}
+
 // DestroyAgent for sorted agent t: the slot keeps the state it is destroyed
 // with: step-start position and velocity, this step's attraction point, the
 // previous step's preferred and ORCA velocities (already there after a step
-// that started from the slot arrays).  Appends the event and fences it.
+// that started from the slot arrays).
 __device__ __forceinline__ void retire_agent(const DevState& s, const AttrIn& in, V2 attr) {
     const int id = __float_as_int(in.pr.w);
     s.pos_in[id] = make_float2(in.pr.x, in.pr.y);
@@ -828,15 +891,12 @@ __device__ __forceinline__ void retire_agent(const DevState& s, const AttrIn& in
         if (s.v_orca) s.v_orca[id] = s.v_orca_s_old[in.prev];
     }
     s.active[id] = 0;
-    const uint32_t q = atomicAdd(s.events_n, 1u);
-    s.events[q] = make_int4(id, 0, 0, -1);
-    __threadfence();
+    put_event(s, id, 0, 0, -1);
 }
 
 // The goal check, attraction point and steering of the agent at sorted
-// position t (with the destroy or replan request it may make).  Returns
-// whether it appended an event, after fencing it device-wide.
-__device__ __forceinline__ bool attr_agent(const DevState& s, int t, const AttrIn& in) {
+// position t (with the destroy or replan request it may make).
+__device__ __forceinline__ void attr_agent(const DevState& s, int t, const AttrIn& in) {
     const V2 pos = mk(in.pr.x, in.pr.y);
     const EnvDesc& E = env_of_sorted(s, in.sv);
 
@@ -844,22 +904,23 @@ __device__ __forceinline__ bool attr_agent(const DevState& s, int t, const AttrI
     const int np = in.pc.y;
     const float2* path = s.path_pts + in.pc.x;
     float2 gg = path[np - 1];
+    // for every agent, so that its loads go out with the goal's
+    uint32_t fb = 0;
+    const int cell = locate_cell(E, pos, fb);
     float gx = pos.x - gg.x, gy = pos.y - gg.y;
     float dGoal = gx * gx + gy * gy;
     V2 attr = mk(in.a0.x, in.a0.y);
-    bool alive = true, event = false;
-    uint32_t fb = 0;
+    bool alive = true;
     if (dGoal < s.arrival_r2) {
         attr = mk(gg.x, gg.y);
         if (dGoal < s.delete_r2) alive = false;
+        fb = 0;
     } else {
         V2 ap = mk(0.0f, 0.0f);
-        if (irm_attraction(E, pos, path, np, ap, fb)) attr = ap;
+        if (irm_attraction(E, pos, cell, path, np, ap)) attr = ap;
         else {
             // UpdatePath(e, currentPosition, goal) with the step-start position
-            uint32_t q = atomicAdd(s.events_n, 1u);
-            s.events[q] = make_int4(__float_as_int(in.pr.w), __float_as_int(pos.x), __float_as_int(pos.y), t);
-            event = true;
+            put_event(s, __float_as_int(in.pr.w), __float_as_int(pos.x), __float_as_int(pos.y), t);
         }
     }
     s.attr_s[t] = make_float2(attr.x, attr.y);
@@ -867,14 +928,12 @@ __device__ __forceinline__ bool attr_agent(const DevState& s, int t, const AttrI
     s.dead_s[t] = alive ? 0 : 1;
     if (!alive) {
         retire_agent(s, in, attr);
-        return true;
+        return;
     }
     // ApplySteeringForce (Simulator.cpp:638-657)
     const float speed = in.sv.z;
     V2 des = normalize(attr - pos) * speed;
     s.pref_vel_s[t] = make_float2(des.x, des.y);
-    if (event) __threadfence();
-    return event;
 }
 
 // The k nearest of sorted agent t (replaces KDTree::KNearestAgents); an
@@ -907,22 +966,23 @@ __device__ __forceinline__ void knn_agent(const DevState& s, int* knn_lds, int t
     s.nbr_cnt[t] = cnt;
 }
 
-// The block that finishes last copies the step's counters and its first
-// event_peek events (words [0, 8 + 4 * min(events, peek)) of the block that
-// events_n heads) to host_xfer[1..], then, after a system-scope fence, the
-// step number (acc[12]) to host_xfer[0]: the host polls that word and reads
-// the rest once it matches.  Only the threads that appended an event fence
-// (device scope, before the block barrier), so the rare events cost the
-// rare fences; an agent-scope fence in every block would write back its
-// XCD's L2 each time.  The last block reads with device-scope atomic loads.
-__device__ __forceinline__ void publish_if_last(const DevState& s) {
+// The last of `blocks` blocks to finish copies the step's counters and its
+// first event_peek events (words [0, 8 + 4 * min(events, peek)) of the block
+// that events_n heads) to host_xfer[1..], then the step number (acc[12]) to
+// host_xfer[0]: the host polls that word and reads the rest once it matches.
+// No fence: the events were stored past the L2 (put_event) and are loaded past
+// it, the host's words are stored at system scope and waited for before the
+// step number goes out.  A system fence writes back the XCD's L2 first, and
+// two of them, with the one before the loads, stood at the end of every
+// launch.
+__device__ __forceinline__ void publish_if_last(const DevState& s, uint32_t blocks) {
     __shared__ uint32_t last;
     __syncthreads();
     if (threadIdx.x == 0) {
         // through kDoneGroups counters first: one address takes an atomic
         // each 20-30 ns, and a million agents have 3,700 blocks
         bool l = true;
-        uint32_t n = gridDim.x;
+        uint32_t n = blocks;
         if (n > 2 * kDoneGroups) {
             const uint32_t g = blockIdx.x % kDoneGroups;
             uint32_t* at = s.group_done + g * kStatStride;
@@ -934,19 +994,18 @@ __device__ __forceinline__ void publish_if_last(const DevState& s) {
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();
     const uint32_t* xfer = s.events_n;
     const uint32_t ne = __hip_atomic_load(xfer, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t n = 8u + 4u * min(ne, s.event_peek);
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
-        s.host_xfer[1 + i] = __hip_atomic_load(xfer + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __threadfence_system();
+        __hip_atomic_store(s.host_xfer + 1 + i, __hip_atomic_load(xfer + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    stores_done();
     __syncthreads();
     if (threadIdx.x == 0) {
         *s.blocks_done = 0u;
         s.acc[15] = 0;                       // every block's grid build has used it
-        __threadfence_system();
-        *(volatile uint32_t*)s.host_xfer = (uint32_t)s.acc[12];
+        __hip_atomic_store(s.host_xfer, (uint32_t)s.acc[12], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -958,15 +1017,23 @@ __device__ __forceinline__ void publish_if_last(const DevState& s) {
 __global__ __launch_bounds__(256) void k_attr(DevState s) {
     const int t = xcd_block() * blockDim.x + threadIdx.x;
     if (t < (int)s.cell_start[s.n_keys]) attr_agent(s, t, attr_in(s, t));
-    publish_if_last(s);
+    publish_if_last(s, gridDim.x);
 }
 
 // An element of a build from the last step's sorted outputs: agent t of the
-// last step, or the (t - n_old)-th agent spawned since.  Stores its state at
-// its sorted position `slot` with the maps between the two orders for the
-// neighbour seeds, and returns it.
-__device__ __forceinline__ AttrIn scatter_agent(const DevState& s, int t, int n_old, int slot, bool write) {
+// last step, or the (t - n_old)-th agent spawned since.
+struct Moved {
+    uint32_t m;          // its cell, kInvalidKey: none
+    uint32_t in_cell;    // its place from the start of the cell's scan block
     AttrIn in;
+};
+__device__ __forceinline__ Moved moved_agent(const DevState& s, int t, int n_old, int n) {
+    Moved M;
+    M.m = kInvalidKey;
+    if (t >= n) return M;
+    M.m = s.key[t];
+    const uint32_t rank = s.rank[t];
+    AttrIn& in = M.in;
     if (t >= n_old) {                                  // spawned since the last step: no seeds
         const int id = s.new_ids[t - n_old];
         const float2 p = s.pos_in[id], v = s.vel_in[id];
@@ -983,36 +1050,40 @@ __device__ __forceinline__ AttrIn scatter_agent(const DevState& s, int t, int n_
         in.a0 = s.attr_s_old[t];
         in.pc = s.path_s_old[t];
         in.prev = t;
-        if (write) s.fwd[t] = slot;
     }
-    if (write) {
-        s.sorted_pr[slot] = in.pr;
-        s.sorted_v[slot] = in.sv;
-        s.path_s[slot] = in.pc;
-        s.prev_of[slot] = in.prev;
-    }
-    return in;
+    M.in_cell = M.m == kInvalidKey ? 0u : s.cell_local[M.m] + rank;
+    return M;
+}
+// Its state at its sorted position, with the maps between the two orders for
+// the neighbour seeds.
+__device__ __forceinline__ void store_moved(const DevState& s, const AttrIn& in, int slot) {
+    if (in.prev >= 0) s.fwd[in.prev] = slot;
+    s.sorted_pr[slot] = in.pr;
+    s.sorted_v[slot] = in.sv;
+    s.path_s[slot] = in.pc;
+    s.prev_of[slot] = in.prev;
 }
 
 // Counting-sort scatter from the last step's sorted outputs, and the
 // attraction pass on what it holds in registers: reads and writes both
 // follow the Morton order, which barely changes from step to step.  One
 // kernel instead of two: the attraction pass does not read back 52 B per
-// agent, and the scatter's stores go out behind its dependent loads.  The
-// last block publishes the events, as in k_attr.
-__global__ __launch_bounds__(256) void k_scatter_attr(DevState s) {
-    __shared__ uint32_t top[kTopMax];
-    const Starts S = scatter_starts(s, top);
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
+// agent, and the scatter's stores go out behind its dependent loads.  An
+// agent's loads go out before the block totals are scanned.  The last block
+// publishes the events, as in k_attr.
+__global__ __launch_bounds__(256) void k_scatter_attr(DevState s, uint32_t blocks) {
+    __shared__ __align__(16) uint32_t top[kTopMax];
+    if (blockIdx.x >= blocks) { write_starts(s, blockIdx.x - blocks); return; }
+    const int t = xcd_block((int)blocks) * blockDim.x + threadIdx.x;
     const int n_old = (int)(uint32_t)s.acc[14];
-    if (t < n_old + (int)(uint32_t)s.acc[15]) {
-        const uint32_t m = s.key[t];
-        if (m != kInvalidKey) {
-            const int slot = (int)(S.at(m) + s.rank[t]);
-            attr_agent(s, slot, scatter_agent(s, t, n_old, slot, true));
-        }
+    const Moved M = moved_agent(s, t, n_old, n_old + (int)(uint32_t)s.acc[15]);
+    const Starts S = scatter_starts(s, top);
+    if (M.m != kInvalidKey) {
+        const int slot = (int)(S.pre[M.m / kScanCells] + M.in_cell);
+        store_moved(s, M.in, slot);
+        attr_agent(s, slot, M.in);
     }
-    publish_if_last(s);
+    publish_if_last(s, blocks);
 }
 
 // The k nearest of every agent (kKnnBuf + 2 kKnnRanges ints of LDS per lane).
@@ -1759,11 +1830,10 @@ __global__ __launch_bounds__(64) void k_orca(DevState s) {
 // nObst slots, in scan order) and the K agent constraints, RandomizedLP
 // over them (lp2_reg), then integration or the 3D-LP queue.  An agent with
 // more than OB obstacle constraints is parked untouched for k_orca_ovf.
-// At K 10 and OB 4 the pass is capped at 80 VGPRs for 6 waves per SIMD: a
-// small spill (68 B per lane) costs less than the latency the sixth wave
-// hides (ORCA phase 0.45 -> 0.42 ms at c2's dense window; 7 and 8 waves
-// spill 156 and 192 B and are slower).
-constexpr int orca_reg_waves(int K, int OB) { return K <= 10 && OB <= 4 ? 6 : 1; }
+// At K 10 and OB 4 the pass is capped at 96 VGPRs for 5 waves per SIMD, which
+// need no spill (950,000 jammed agents, k_knn_orca: 5 waves 269 us; 6 waves
+// spill 84 B per lane: 299, or 28 B with the branching half-planes: 283).
+constexpr int orca_reg_waves(int K, int OB) { return K <= 10 && OB <= 4 ? 5 : 1; }
 
 template <int K, int OB>
 __device__ __forceinline__ void orca_reg_agent(const DevState& s, int t);
@@ -1782,7 +1852,7 @@ __global__ __launch_bounds__(64, orca_reg_waves(K, OB)) void k_orca_reg(DevState
 // neighbour list and preferred velocity, so no other thread's result is
 // waited for.  One kernel instead of two: the neighbour list is read back
 // from the thread's own writes, and the tail of one pass overlaps the
-// other's.  Capped at 80 VGPRs for 6 waves per SIMD.
+// other's.  Capped at 96 VGPRs for 5 waves per SIMD (orca_reg_waves).
 // k_knn_orca for small crowds: 16 agents per 64-lane wavefront.  A crowd
 // of a few thousand agents fills a few dozen wavefronts, one per SIMD, and
 // the pass lasts as long as one wavefront's walk, constraints and LP; with
@@ -1803,7 +1873,7 @@ __global__ __launch_bounds__(64, 6) void k_knn_orca_sparse(DevState s) {
 }
 
 template <int K>
-__global__ __launch_bounds__(256, 6) void k_knn_orca(DevState s) {
+__global__ __launch_bounds__(256, 5) void k_knn_orca(DevState s) {
     extern __shared__ int knn_lds[];
     const uint32_t n_active = s.cell_start[s.n_keys];
     const int t = xcd_block() * blockDim.x + threadIdx.x;
@@ -1858,9 +1928,7 @@ __device__ __forceinline__ void orca_reg_agent(const DevState& s, int t) {
     uint32_t aval = 0u, redo = 0u;
     // the neighbours' loads in batches of kNbrBatch, each batch issued before
     // its constraints are built: the loads of a batch are in flight together,
-    // and the batch's 6 registers per neighbour stay within the 80-VGPR cap
-    // (all 10 at once spilled 68 B per lane; two batches of 5 spill 24 B and
-    // took the pass from 0.263 to 0.238 ms at c2's jam)
+    // and the batch's 6 registers per neighbour stay within the register cap
     constexpr int kNbrBatch = (K + 1) / 2;
 #pragma unroll
     for (int h = 0; h < K; h += kNbrBatch) {
@@ -2219,10 +2287,10 @@ hipError_t launch_grid_attr(const DevState& s, bool row, int n_cu, hipStream_t s
     if (nb > kTopMax) hipLaunchKernelGGL(k_scan_top, dim3(1), b, 0, st, s.bsum, nb, s.cell_start, s.n_keys, s.acc + 13);
     if (mid && s.sorted_in) (void)hipEventRecord(mid, st);
     if (s.sorted_in) {
-        if (row) hipLaunchKernelGGL(k_scatter_attr_row, gr, b, 0, st, s);
-        else hipLaunchKernelGGL(k_scatter_attr, ga, b, 0, st, s);
+        if (row) hipLaunchKernelGGL(k_scatter_attr_row, dim3(gr.x + nb), b, 0, st, s, gr.x);
+        else hipLaunchKernelGGL(k_scatter_attr, dim3(ga.x + nb), b, 0, st, s, ga.x);
     } else {
-        hipLaunchKernelGGL(k_grid_scatter, ga, b, 0, st, s);
+        hipLaunchKernelGGL(k_grid_scatter, dim3(ga.x + nb), b, 0, st, s, ga.x);
         if (mid) (void)hipEventRecord(mid, st);
         if (row) hipLaunchKernelGGL(k_attr_row, gr, b, 0, st, s);
         else hipLaunchKernelGGL(k_attr, ga, b, 0, st, s);
