@@ -72,9 +72,9 @@ struct ecm_mlp {
     ecm::DBuf<float2> ds_v;        // [cap]
     ecm::DBuf<uint32_t> ds_count;  // [1] device append counter
     int64_t ds_cap = 0;
-    // BF16 features of the last host batch (kept: a fresh buffer costs a page
-    // fault per 4 KiB in every call)
-    std::vector<uint16_t> h_x;
+    // page-locked staging of host batches and results, kStageBytes from the
+    // first call on that uses it
+    unsigned char* stage = nullptr;
     // staged host batch, for batch size in_batch
     int in_batch = 0;
     ecm::DBuf<bf16x8_t> xb;
