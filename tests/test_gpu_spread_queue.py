@@ -4,7 +4,8 @@ block totals a scatter block scans one per thread, eight per thread or finds
 scanned, give the same states, neighbours and statistics, bit for bit, as the
 row step or a coarse grid; agents whose half-planes the branch-free form does
 not cover (no radius, T off the powers of two) match the oracle; and host
-batches around the staging's pieces give the network's rows."""
+batches around the staging's pieces give the network's rows.  A step with more
+events than the host block holds delivers them all."""
 import numpy as np
 import pytest
 
@@ -104,3 +105,28 @@ def test_staged_batches(n):
     y = net.forward(x)
     for a in (0, max(0, n // 2 - 100), max(0, n - 300)):
         assert np.array_equal(y[a:a + 300], net.forward(np.ascontiguousarray(x[a:a + 300])))
+
+
+@pytest.mark.parametrize("shape", [256, 64])
+def test_more_events_than_the_host_block_holds(shape):
+    """1,500 agents at their goals beside 500 that walk: the events past the
+    host block's 1,024 are copied from the device's list."""
+    rng = np.random.default_rng(9)
+    n, gone = 2000, 1500
+    start = rng.uniform(-60.0, 60.0, (n, 2)).astype(np.float32)
+    off = np.where(np.arange(n)[:, None] < gone, 0.5, 40.0).astype(np.float32)
+    path = np.stack([start, start + off], 1).reshape(-1, 2).astype(np.float32)
+    agents = Agents(start, np.full(n, 0.2, np.float32), np.full(n, 1.3, np.float32),
+                    np.arange(n, dtype=np.int32) * 2, np.full(n, 2, np.int32), path)
+    box = (-120.0, -120.0, 120.0, 120.0)
+    _, _, obs, _, _ = small_scene(3, half=100.0, n_rects=1, n_agents=1, side=(1, 2))
+    sim = Simulator(square(box), obs, box, Params(max_agents=n))
+    ids = sim.SpawnAgents(agents, validate=False)
+    sim.set_tuning(knn_block=shape)
+    sim.Update(steps=3)
+    active = sim.state()["active"].astype(bool)
+    assert not active[ids[:gone]].any() and active[ids[gone:]].all()
+    again = sim.SpawnAgents(Agents(start[:gone], agents.radius[:gone], agents.pref_speed[:gone], agents.path_off[:gone],
+                                   agents.path_cnt[:gone], path), validate=False)
+    assert np.array_equal(np.sort(again), np.sort(ids[:gone]))
+    sim.close()
