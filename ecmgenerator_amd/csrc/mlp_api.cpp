@@ -357,11 +357,13 @@ extern "C" int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y) {
 }
 
 // ------------------------------------------- forward without allocation
-// Scratch of ecm_mlp_forward_noalloc: the proposal masks ([n]) of up to
+// Scratch of ecm_mlp_forward_noalloc: the proposal masks ([n]) and the output
+// rows ([n][16] FP32, for a y that overlaps x) of up to
 // ECM_MLP_NOALLOC_MAX_SAMPLES samples.  Every GPU holds its own copy until
 // the process ends.  Nothing in it has to start at zero: the network writes
-// every mask.
-constexpr size_t kNoAllocBytes = (size_t)ECM_MLP_NOALLOC_MAX_SAMPLES * 4;
+// every mask and every row.
+constexpr size_t kNoAllocMaskBytes = (size_t)ECM_MLP_NOALLOC_MAX_SAMPLES * 4;
+constexpr size_t kNoAllocBytes = kNoAllocMaskBytes + (size_t)ECM_MLP_NOALLOC_MAX_SAMPLES * kOut * 4;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
 // Device address of `scratch` on device `dev`, looked up once per device
@@ -392,9 +394,15 @@ extern "C" int ecm_mlp_forward_noalloc(ecm_mlp* m, const float* x, int n, float*
     int rc = scratch_address(m->dev, &base);
     if (rc) return rc;
     // the network reads the FP32 rows itself, rounding as the host staging of
-    // ecm_mlp_forward does
+    // ecm_mlp_forward does; output rows over its input rows would reach tiles
+    // that are yet to be read, and wait in the scratch
+    const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+    const size_t in_bytes = (size_t)n * kInPad * 4, out_bytes = (size_t)n * kOut * 4;
+    const bool overlap = x0 < y0 + out_bytes && y0 < x0 + in_bytes;
+    float* out = overlap ? reinterpret_cast<float*>(base + kNoAllocMaskBytes) : y;
     HIPCHK(launch_mlp_infer(x, 2, nullptr, n, m->frags.p, m->pbias.p, 0.0f, reinterpret_cast<uint32_t*>(base), nullptr,
-                            y, m->n_cu, m->stream));
+                            out, m->n_cu, m->stream));
+    if (overlap) HIPCHK(launch_copy_f32(y, out, (long)n * kOut, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
     return 0;
 }

@@ -47,6 +47,7 @@ inline int train_chunks(int n) { return n <= 128 ? 1 : (n >= 96 * 128 ? 96 : (n 
 hipError_t launch_train_pack(const float* params, void* frags, hipStream_t st);
 hipError_t launch_train_batch(const TrainBatch& t, hipStream_t st);
 hipError_t launch_fill_f32(float* p, float v, long n, hipStream_t st);
+hipError_t launch_copy_f32(float* to, const float* from, long n, hipStream_t st);
 hipError_t launch_pack(const float* P, void* frags, float* bias, hipStream_t st);
 
 }  // namespace mlp

@@ -584,6 +584,10 @@ __global__ void k_fill_f32(float* p, float v, long n) {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = v;
 }
 
+__global__ void k_copy_f32(float* to, const float* from, long n) {
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) to[i] = from[i];
+}
+
 // Inference packing of the FP32 parameters (fragment layout in mlp.h).
 __global__ void k_pack(const float* P, bf16x8* frags, float* bias) {
     const int f = blockIdx.x, lane = threadIdx.x;          // one fragment per block, 64 lanes
@@ -656,6 +660,12 @@ hipError_t launch_train_batch(const TrainBatch& t, hipStream_t st) {
 hipError_t launch_fill_f32(float* p, float v, long n, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_fill_f32, dim3(std::min(cdiv(n, 256), 4096)), dim3(256), 0, st, p, v, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_f32(float* to, const float* from, long n, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_copy_f32, dim3(std::min(cdiv(n, 256), 4096)), dim3(256), 0, st, to, from, n);
     return hipGetLastError();
 }
 

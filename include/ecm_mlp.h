@@ -77,8 +77,9 @@ int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y);
 /* ecm_mlp_forward for device buffers, allocating nothing: x (n*64 FP32)
  * and y (n*16 raw outputs) are device memory of the handle's GPU, and the
  * proposal masks go to a static scratch array of the library (one per GPU,
- * ECM_MLP_NOALLOC_MAX_SAMPLES samples = 128 KiB, held until the process
- * ends).  No hipMalloc, hipFree or other allocating
+ * ECM_MLP_NOALLOC_MAX_SAMPLES samples = 2.125 MiB, held until the process
+ * ends).  y may lie over x: its rows then wait in the scratch until the
+ * network has read all of x.  No hipMalloc, hipFree or other allocating
  * call; n above the maximum is rejected with ECM_E_ARG.  Calls that
  * overlap on one GPU share the scratch and race.  Returns after y is
  * written.  No counterpart in the reference: it is for callers that cannot
