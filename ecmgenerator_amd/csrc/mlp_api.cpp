@@ -2,6 +2,7 @@
 // dataset, the training loop (forward, backward and Adam on the GPU with
 // the kernels of mlp_kernels.hip) and host-data entry points.
 #include "mlp_host.h"
+#include "stage.h"
 
 #include <algorithm>
 #include <cmath>
@@ -257,11 +258,9 @@ static TrainBatch train_batch(ecm_mlp* m, int B, float pos_w, float vel_w) {
     return t;
 }
 
-// Host batches go through page-locked memory piece by piece, each piece's copy
-// running while the next is rounded; results of up to kStageBytes come back
-// through it.  Pageable buffers are copied by the runtime into memory of its
-// own first, piece by piece with waits between, and its first touch of each
-// result waits again.
+// Host batches go through page-locked memory piece by piece (stage.h); results
+// of up to kStageBytes come back through it, since the runtime's first touch
+// of each result in pageable memory waits again.
 constexpr size_t kStagePiece = 256 << 10, kStagePieces = 16, kStageBytes = kStagePieces * kStagePiece;
 
 static int ensure_stage(ecm_mlp* m) {
@@ -273,50 +272,36 @@ static int ensure_stage(ecm_mlp* m) {
     return 0;
 }
 
-// Staged pieces of one call; the stream is waited for before a piece's memory
-// is used again.  fill(to, at, bytes) writes bytes [at, at + bytes).
-struct Stager {
-    ecm_mlp* m;
-    size_t piece = 0;
-    template <typename F>
-    int put(void* dst, size_t bytes, F&& fill) {
-        for (size_t at = 0; at < bytes; at += kStagePiece, ++piece) {
-            if (piece && piece % kStagePieces == 0) HIPCHK(hipStreamSynchronize(m->stream));
-            unsigned char* to = m->stage + piece % kStagePieces * kStagePiece;
-            const size_t len = std::min(kStagePiece, bytes - at);
-            fill(to, at, len);
-            HIPCHK(hipMemcpyAsync((unsigned char*)dst + at, to, len, hipMemcpyHostToDevice, m->stream));
-        }
+struct StageQueue {
+    hipStream_t st;
+    int copy(void* dst, const void* src, size_t bytes) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
         return 0;
     }
-    int put(void* dst, const void* src, size_t bytes) {
-        return put(dst, bytes, [&](void* to, size_t at, size_t len) { std::memcpy(to, (const unsigned char*)src + at, len); });
+    int wait() {
+        HIPCHK(hipStreamSynchronize(st));
+        return 0;
     }
 };
+using BatchStager = Stager<StageQueue>;
 
-static int stage_host_batch(ecm_mlp* m, const float* x, const uint32_t* label, const float* v, int n) {
-    int rc = ensure_stage(m);
-    if (rc) return rc;
-    Stager st{m};
-    rc = st.put(m->xb.p, (size_t)n * 128, [&](void* to, size_t at, size_t len) {
+static int stage_host_batch(ecm_mlp* m, BatchStager& st, const float* x, const uint32_t* label, const float* v, int n) {
+    int rc = st.put(m->xb.p, (size_t)n * 128, [&](void* to, size_t at, size_t len) {
         round_rows(x + at / 2, (uint16_t*)to, len / 2);
     });
     if (!rc && label) rc = st.put(m->lb.p, label, (size_t)n * 4);
     if (!rc && v) rc = st.put(m->vb.p, v, (size_t)n * 8);
-    return rc;                                    // every caller waits for the stream before it returns
+    return rc;
 }
 
 // The result of a call: `bytes` of device memory, copied into the staging
 // memory once the stream is there, or straight to the caller's when larger.
-static int fetch(ecm_mlp* m, const void* dev, size_t bytes, void* out) {
-    if (bytes <= kStageBytes) {
-        HIPCHK(hipMemcpyAsync(m->stage, dev, bytes, hipMemcpyDeviceToHost, m->stream));
-        HIPCHK(hipStreamSynchronize(m->stream));
-        std::memcpy(out, m->stage, bytes);
-        return 0;
-    }
-    HIPCHK(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, m->stream));
+static int fetch(ecm_mlp* m, BatchStager& st, const void* dev, size_t bytes, void* out) {
+    const bool staged = bytes <= kStageBytes;
+    HIPCHK(hipMemcpyAsync(staged ? (void*)m->stage : out, dev, bytes, hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
+    st.waited();
+    if (staged) std::memcpy(out, m->stage, bytes);
     return 0;
 }
 
@@ -326,8 +311,11 @@ extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* lab
     (void)hipSetDevice(m->dev);
     int rc = ensure_ws(m, n);
     if (!rc) rc = ensure_in(m, n);
-    if (!rc) rc = stage_host_batch(m, x, label, v, n);
-    if (rc) { (void)hipStreamSynchronize(m->stream); return rc; }
+    if (!rc) rc = ensure_stage(m);
+    if (rc) return rc;
+    StageQueue q{m->stream};
+    BatchStager st(q, m->stage, kStagePiece, kStagePieces);
+    if ((rc = stage_host_batch(m, st, x, label, v, n)) != 0) return rc;
     if ((rc = pack_train(m)) != 0) return rc;
     TrainBatch t = train_batch(m, n, pos_weight, vel_weight);
     t.first = true;
@@ -340,6 +328,7 @@ extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* lab
     static_assert((kNParams + 1) * sizeof(float) <= kStageBytes, "one fetch");
     HIPCHK(hipMemcpyAsync(m->stage, m->grads.p, (kNParams + 1) * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
+    st.waited();
     std::memcpy(grad, m->stage, kNParams * sizeof(float));
     std::memcpy(loss, m->stage + kNParams * sizeof(float), sizeof(float));
     return 0;
@@ -349,11 +338,14 @@ extern "C" int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y) {
     if (!m || !x || !y || n < 1) return fail(ECM_E_ARG, "bad arguments");
     (void)hipSetDevice(m->dev);
     int rc = ensure_in(m, n);
-    if (!rc) rc = stage_host_batch(m, x, nullptr, nullptr, n);
-    if (rc) { (void)hipStreamSynchronize(m->stream); return rc; }
+    if (!rc) rc = ensure_stage(m);
+    if (rc) return rc;
+    StageQueue q{m->stream};
+    BatchStager st(q, m->stage, kStagePiece, kStagePieces);
+    if ((rc = stage_host_batch(m, st, x, nullptr, nullptr, n)) != 0) return rc;
     HIPCHK(launch_mlp_infer(m->xb.p, 0, nullptr, n, m->frags.p, m->pbias.p, 0.0f, m->lb.p, nullptr, m->y.p, m->n_cu,
                             m->stream));
-    return fetch(m, m->y.p, (size_t)n * kOut * sizeof(float), y);
+    return fetch(m, st, m->y.p, (size_t)n * kOut * sizeof(float), y);
 }
 
 // ------------------------------------------- forward without allocation
