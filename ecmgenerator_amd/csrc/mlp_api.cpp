@@ -7,7 +7,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <random>
 #include <vector>
 
@@ -259,18 +261,37 @@ static TrainBatch train_batch(ecm_mlp* m, int B, float pos_w, float vel_w) {
 }
 
 // Host batches go through page-locked memory piece by piece (stage.h); results
-// of up to kStageBytes come back through it, since the runtime's first touch
+// that fit into it come back through it, since the runtime's first touch
 // of each result in pageable memory waits again.
-constexpr size_t kStagePiece = 256 << 10, kStagePieces = 16, kStageBytes = kStagePieces * kStagePiece;
+constexpr size_t kStagePiece = 256 << 10, kStagePieces = 16;
 
-static int ensure_stage(ecm_mlp* m) {
-    if (m->stage) return 0;
-    if (hipHostMalloc((void**)&m->stage, kStageBytes, hipHostMallocDefault) != hipSuccess) {
-        m->stage = nullptr;
-        return fail(ECM_E_HIP, "hipHostMalloc of %zu bytes failed", kStageBytes);
+// What a host call of n rows is staged through: the handle's page-locked
+// pieces or, in a first call of few rows, ordinary memory with a piece for each
+// of the three arrays.
+struct Stage {
+    unsigned char* mem = nullptr;
+    size_t piece = kStagePiece, pieces = kStagePieces;
+    std::unique_ptr<unsigned char[]> own;
+    int open(ecm_mlp* m, size_t n) {
+        const bool first = !m->host_called;
+        m->host_called = true;
+        if (!m->stage && !stage_page_locked(first, n)) {
+            own.reset(new (std::nothrow) unsigned char[kFirstCallRows * 128 * 3]);
+            if (own) {
+                mem = own.get();
+                piece = kFirstCallRows * 128;
+                pieces = 3;
+                return 0;
+            }
+        }
+        if (!m->stage && hipHostMalloc((void**)&m->stage, piece * pieces, hipHostMallocDefault) != hipSuccess) {
+            m->stage = nullptr;
+            return fail(ECM_E_HIP, "hipHostMalloc of %zu bytes failed", piece * pieces);
+        }
+        mem = m->stage;
+        return 0;
     }
-    return 0;
-}
+};
 
 struct StageQueue {
     hipStream_t st;
@@ -296,12 +317,12 @@ static int stage_host_batch(ecm_mlp* m, BatchStager& st, const float* x, const u
 
 // The result of a call: `bytes` of device memory, copied into the staging
 // memory once the stream is there, or straight to the caller's when larger.
-static int fetch(ecm_mlp* m, BatchStager& st, const void* dev, size_t bytes, void* out) {
-    const bool staged = bytes <= kStageBytes;
-    HIPCHK(hipMemcpyAsync(staged ? (void*)m->stage : out, dev, bytes, hipMemcpyDeviceToHost, m->stream));
+static int fetch(ecm_mlp* m, const Stage& stage, BatchStager& st, const void* dev, size_t bytes, void* out) {
+    const bool staged = bytes <= stage.piece * stage.pieces;
+    HIPCHK(hipMemcpyAsync(staged ? (void*)stage.mem : out, dev, bytes, hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
     st.waited();
-    if (staged) std::memcpy(out, m->stage, bytes);
+    if (staged) std::memcpy(out, stage.mem, bytes);
     return 0;
 }
 
@@ -311,10 +332,11 @@ extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* lab
     (void)hipSetDevice(m->dev);
     int rc = ensure_ws(m, n);
     if (!rc) rc = ensure_in(m, n);
-    if (!rc) rc = ensure_stage(m);
+    Stage stage;
+    if (!rc) rc = stage.open(m, n);
     if (rc) return rc;
     StageQueue q{m->stream};
-    BatchStager st(q, m->stage, kStagePiece, kStagePieces);
+    BatchStager st(q, stage.mem, stage.piece, stage.pieces);
     if ((rc = stage_host_batch(m, st, x, label, v, n)) != 0) return rc;
     if ((rc = pack_train(m)) != 0) return rc;
     TrainBatch t = train_batch(m, n, pos_weight, vel_weight);
@@ -325,12 +347,12 @@ extern "C" int ecm_mlp_loss_grad(ecm_mlp* m, const float* x, const uint32_t* lab
     t.grad = m->grads.p;
     HIPCHK(launch_train_batch(t, m->stream));
     // the loss stands behind the gradient
-    static_assert((kNParams + 1) * sizeof(float) <= kStageBytes, "one fetch");
-    HIPCHK(hipMemcpyAsync(m->stage, m->grads.p, (kNParams + 1) * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    static_assert((kNParams + 1) * sizeof(float) <= 3 * kFirstCallRows * 128, "one fetch");
+    HIPCHK(hipMemcpyAsync(stage.mem, m->grads.p, (kNParams + 1) * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
     st.waited();
-    std::memcpy(grad, m->stage, kNParams * sizeof(float));
-    std::memcpy(loss, m->stage + kNParams * sizeof(float), sizeof(float));
+    std::memcpy(grad, stage.mem, kNParams * sizeof(float));
+    std::memcpy(loss, stage.mem + kNParams * sizeof(float), sizeof(float));
     return 0;
 }
 
@@ -338,14 +360,15 @@ extern "C" int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y) {
     if (!m || !x || !y || n < 1) return fail(ECM_E_ARG, "bad arguments");
     (void)hipSetDevice(m->dev);
     int rc = ensure_in(m, n);
-    if (!rc) rc = ensure_stage(m);
+    Stage stage;
+    if (!rc) rc = stage.open(m, n);
     if (rc) return rc;
     StageQueue q{m->stream};
-    BatchStager st(q, m->stage, kStagePiece, kStagePieces);
+    BatchStager st(q, stage.mem, stage.piece, stage.pieces);
     if ((rc = stage_host_batch(m, st, x, nullptr, nullptr, n)) != 0) return rc;
     HIPCHK(launch_mlp_infer(m->xb.p, 0, nullptr, n, m->frags.p, m->pbias.p, 0.0f, m->lb.p, nullptr, m->y.p, m->n_cu,
                             m->stream));
-    return fetch(m, st, m->y.p, (size_t)n * kOut * sizeof(float), y);
+    return fetch(m, stage, st, m->y.p, (size_t)n * kOut * sizeof(float), y);
 }
 
 // ------------------------------------------- forward without allocation

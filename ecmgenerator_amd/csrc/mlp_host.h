@@ -73,9 +73,10 @@ struct ecm_mlp {
     ecm::DBuf<float2> ds_v;        // [cap]
     ecm::DBuf<uint32_t> ds_count;  // [1] device append counter
     int64_t ds_cap = 0;
-    // page-locked staging of host batches and results, kStageBytes from the
-    // first call on that uses it
+    // page-locked staging of host batches and results, 4 MiB from the first
+    // call on that goes through it (stage_page_locked)
     unsigned char* stage = nullptr;
+    bool host_called = false;
     // staged host batch, for batch size in_batch
     int in_batch = 0;
     ecm::DBuf<bf16x8_t> xb;

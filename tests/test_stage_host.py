@@ -90,3 +90,27 @@ def test_no_call_ends_with_copies_in_flight():
         r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
         assert r.returncode == 0, r.stderr
         assert r.stdout.split() == ["bad", "0", "busy", "0", "left", "0", "extra", "0"]
+
+
+RULE = r"""
+#include "stage.h"
+#include <cstdio>
+int main() {
+    for (bool first : {true, false})
+        for (size_t n : {1, 512, 513, 60000}) printf("%d ", (int)ecm::stage_page_locked(first, n));
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(GXX is None, reason="g++ not found")
+def test_first_call_of_few_rows_allocates_nothing_page_locked():
+    with tempfile.TemporaryDirectory() as d:
+        src = os.path.join(d, "rule.cpp")
+        exe = os.path.join(d, "rule")
+        with open(src, "w") as f:
+            f.write(RULE)
+        subprocess.run([GXX, "-O2", "-std=c++17", "-I", CSRC, src, "-o", exe], check=True)
+        r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr
+        assert r.stdout.split() == ["0", "0", "1", "1"] + ["1"] * 4
