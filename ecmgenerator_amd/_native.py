@@ -77,6 +77,7 @@ SIGNATURES = {
     "ecm_sim_stats": (_I, [_P, C.POINTER(C.c_uint64), _I]),
     "ecm_sim_set_graph": (_I, [_P, _I]),
     "ecm_sim_graph_status": (_I, [_P, _PI, C.c_char_p, _I]),
+    "ecm_sim_graph_counts": (_I, [_P, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
     "ecm_sim_get_tuning": (_I, [_P, C.POINTER(SimTuning)]),
     "ecm_sim_set_tuning": (_I, [_P, C.POINTER(SimTuning)]),
     "ecm_sim_autotune": (_I, [_P, _I, C.POINTER(SimTuning)]),

@@ -279,7 +279,8 @@ struct ecm_sim {
         hipGraphExec_t exec[2] = {nullptr, nullptr};
     };
     bool use_graph = false;
-    bool idle = true;                           // nothing queued on the stream since it was last waited for
+    bool idle = true;                           // no step queued on the stream since it was last waited for
+    uint64_t graph_replays = 0, graph_captures = 0;
     bool row_step = false, row_attr = false;    // 16 lanes per agent (row_rule)
     int row_agents = 0;                         // agents their grid is sized for
     StepGraph graphs[2][2];                     // [parity][entry from the sorted outputs]
@@ -610,7 +611,7 @@ static int build_obstacle_buckets(ecm_sim* s, EnvHost* E, float range) {
         HIPCHK(hipMemcpyAsync(E->obucket_start.p, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice, s->stream));
         if (!edges.empty())
             HIPCHK(hipMemcpyAsync(E->obucket_edges.p, edges.data(), edges.size() * sizeof(int), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if (int rc_ = settle(s)) return rc_;
         E->og = g;
         s->envs_dirty = true;
         E->maxo = maxlen <= 16 ? 16 : (maxlen <= 32 ? 32 : (maxlen <= 64 ? 64 : (int)((maxlen + 15) & ~(size_t)15)));
@@ -679,7 +680,7 @@ extern "C" int ecm_sim_env_set_obstacles(ecm_sim* s, int env, const float* xy, c
     HIPCHK(hipMemcpyAsync(E->oe0.p, e0.data(), nv * sizeof(float4), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(E->oe1.p, e1.data(), nv * sizeof(float4), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(E->oe2.p, e2.data(), nv * sizeof(float4), hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     E->obst_range_built = -1.0f;   // (re)bucketed at the next step
     s->envs_dirty = true;
     return 0;
@@ -834,7 +835,7 @@ extern "C" int ecm_sim_env_set_ecm(ecm_sim* s, int env, int n_vert, const float*
     HIPCHK(hipMemcpyAsync(E->yhash_cnt.p, tcnt.data(), tsize * sizeof(int), hipMemcpyHostToDevice, s->stream));
     if (!ycells.empty())
         HIPCHK(hipMemcpyAsync(E->ycells.p, ycells.data(), ycells.size() * sizeof(int), hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     E->eg = g;
     E->yhash_mask = (int)tsize - 1;
     return 0;
@@ -907,7 +908,7 @@ static int ensure_path_capacity(ecm_sim* s, size_t extra) {
     if (hipMalloc((void**)&np, cap * sizeof(float2)) != hipSuccess) return fail(ECM_E_HIP, "path pool growth failed");
     if (s->path_used)
         HIPCHK(hipMemcpyAsync(np, s->path_pool.p, s->path_used * sizeof(float2), hipMemcpyDeviceToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     s->path_pool.release();
     s->path_pool.p = np;
     s->path_pool.n = cap;
@@ -953,7 +954,7 @@ extern "C" int ecm_sim_env_spawn(ecm_sim* s, int env, int n, const float* start_
         if (s->num_agents > 0) {
             cur_pos.resize(s->prm.max_agents);
             HIPCHK(hipMemcpyAsync(cur_pos.data(), s->pos.p, cur_pos.size() * sizeof(float2), hipMemcpyDeviceToHost, s->stream));
-            HIPCHK(hipStreamSynchronize(s->stream));
+            if (int rc_ = settle(s)) return rc_;
             for (int i = 0; i <= s->last_idx; ++i)
                 if (s->h_active[i] && s->h_env[i] == env) hg.add(i, cur_pos[i].x, cur_pos[i].y);
         }
@@ -1035,7 +1036,7 @@ extern "C" int ecm_sim_env_spawn(ecm_sim* s, int env, int n, const float* start_
         HIPCHK(launch_spawn_scatter(n, d_ids.p, d_st.p, d_r.p, d_s.p, d_off.p, d_cnt.p, s->pos.p,
                                     s->vel.p, s->radius.p, s->pref_speed.p, s->pref_vel.p, s->active.p,
                                     s->path_off.p, s->path_cnt.p, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if (int rc_ = settle(s)) return rc_;
     }
     d_ids.release(); d_off.release(); d_cnt.release(); d_st.release(); d_r.release(); d_s.release();
     // the next step keeps entering from the last step's sorted outputs and
@@ -1165,7 +1166,7 @@ extern "C" int ecm_sim_destroy_agent(ecm_sim* s, int id) {
     if (int rc_ = sync_state(s)) return rc_;
     uint8_t z = 0;
     HIPCHK(hipMemcpyAsync(s->active.p + id, &z, 1, hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     mark_destroyed(s, id);
     // an agent spawned since the last step leaves the list of new ones; any
     // other leaves the last step's sorted order (marked destroyed there
@@ -1201,7 +1202,7 @@ extern "C" int ecm_sim_set_path(ecm_sim* s, int id, const float* xy, int n) {
     HIPCHK(hipMemcpyAsync(s->path_pool.p + off, xy, (size_t)n * sizeof(float2), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->path_off.p + id, &off, sizeof(int), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(s->path_cnt.p + id, &n, sizeof(int), hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     s->path_used += (size_t)n;
     s->h_goal[id] = make_float2(xy[2 * (n - 1)], xy[2 * (n - 1) + 1]);
     s->h_path_cnt[id] = n;
@@ -1297,7 +1298,7 @@ static int ensure_agent_grid(ecm_sim* s) {
     rc = zero_dev(s->cell_count.p, GP * sizeof(uint32_t), s->stream);
     if (!rc) rc = zero_dev(s->bsum.p, nb * sizeof(uint32_t), s->stream);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     s->n_keys = (uint32_t)G;
     s->envs_dirty = true;
     return 0;
@@ -1329,13 +1330,13 @@ static int upload_envs(ecm_sim* s) {
             if (rc) return rc;
         }
         HIPCHK(hipMemcpyAsync(s->d_envs.p, h.data(), h.size() * sizeof(EnvDesc), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if (int rc_ = settle(s)) return rc_;
         s->envs_dirty = false;
     }
     if (s->agent_env_dirty) {
         HIPCHK(hipMemcpyAsync(s->agent_env.p, s->h_env.data(), s->h_env.size() * sizeof(uint16_t), hipMemcpyHostToDevice,
                               s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if (int rc_ = settle(s)) return rc_;
         s->agent_env_dirty = false;
     }
     return 0;
@@ -1424,7 +1425,7 @@ static int sync_state(ecm_sim* s) {
     if (s->id_current) return 0;
     const DevState d = make_state(s);        // its "old" arrays are the last step's outputs
     HIPCHK(launch_unsort(d, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     s->id_current = s->pos_current = true;
     return 0;
 }
@@ -1703,6 +1704,7 @@ static int ensure_step_graph(ecm_sim* s, const DevState& d, int mode) {
         }
         g.graph[0] = graph;
         g.exec[0] = exec;
+        ++s->graph_captures;
     }
     g.key = key;
     g.valid = true;
@@ -1730,8 +1732,10 @@ static int step_once(ecm_sim* s) {
         else s->use_graph = false;           // capture refused: eager from now on (see graph_error)
     }
     // the whole step; its first half ends by publishing the events
-    if (graph) HIPCHK(hipGraphLaunch(s->graphs[s->cur][d.sorted_in].exec[0], s->stream));
-    else if ((rc = enqueue_device_half(s, d, mode, 0)) != 0 || (rc = enqueue_device_half(s, d, mode, 1)) != 0)
+    if (graph) {
+        HIPCHK(hipGraphLaunch(s->graphs[s->cur][d.sorted_in].exec[0], s->stream));
+        ++s->graph_replays;
+    } else if ((rc = enqueue_device_half(s, d, mode, 0)) != 0 || (rc = enqueue_device_half(s, d, mode, 1)) != 0)
         return rc;
     s->idle = false;
     const uint32_t peek = (uint32_t)std::min(ecm_sim::kEventPeek, s->prm.max_agents);
@@ -1741,7 +1745,7 @@ static int step_once(ecm_sim* s) {
     if (!ev.empty()) std::memcpy(ev.data(), s->h_xfer + 1 + 8, ev.size() * sizeof(int4));
     if (ne > peek) {
         ev.resize(ne);
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if ((rc = settle(s)) != 0) return rc;
         HIPCHK(hipMemcpy(ev.data() + peek, s->xfer.p + 8 + 4 * (size_t)peek, (ne - peek) * sizeof(int4),
                          hipMemcpyDeviceToHost));
     }
@@ -1791,7 +1795,7 @@ static int step_once(ecm_sim* s) {
     s->stat[4] += nr;
     s->stat[5] += nd;
     if (s->timing) {
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if ((rc = settle(s)) != 0) return rc;
         for (int i = 0; i < 4; ++i) {
             float ms = 0;
             HIPCHK(hipEventElapsedTime(&ms, s->ev[i], s->ev[i + 1]));
@@ -1834,6 +1838,13 @@ extern "C" int ecm_sim_graph_status(ecm_sim* s, int* active, char* why, int cap)
         std::strncpy(why, s->graph_error.c_str(), (size_t)cap - 1);
         why[cap - 1] = 0;
     }
+    return 0;
+}
+
+extern "C" int ecm_sim_graph_counts(ecm_sim* s, uint64_t* replays, uint64_t* captures) {
+    if (!s || !replays || !captures) return fail(ECM_E_ARG, "null argument");
+    *replays = s->graph_replays;
+    *captures = s->graph_captures;
     return 0;
 }
 
@@ -1880,10 +1891,12 @@ extern "C" int ecm_sim_autotune(ecm_sim* s, int steps, ecm_sim_tuning* out) {
         if (!s->envs[e]->ecm_set) return fail(ECM_E_STATE, "set_ecm must be called before autotune (environment %zu)", e);
     (void)hipSetDevice(s->dev);
     if (int rc_ = settle(s)) return rc_;
-    // One sample of a shape: two untimed steps after switching to it (they
-    // recapture the step graphs of both buffer parities), then one step
+    // One sample of a shape: two untimed steps after switching to it (with
+    // graphs on they recapture those of both buffer parities, which only a
+    // step that finds the stream idle does: each is waited for), then one step
     // timed from an idle stream to an idle stream (the device work and the
-    // host's part: events, replans).  The options of a coordinate are
+    // host's part: events, replans), as a program runs it that reads the
+    // state after every step.  The options of a coordinate are
     // sampled round robin, `steps` rounds, and compared by their median: the
     // crowd moves on while the search runs, and round robin spreads that
     // drift over every option.
@@ -1891,11 +1904,9 @@ extern "C" int ecm_sim_autotune(ecm_sim* s, int steps, ecm_sim_tuning* out) {
         apply_tuning(s, t);
         int rc = 0;
         for (int w = 0; w < 2; ++w)
-            if ((rc = step_once(s)) != 0) return rc;
-        HIPCHK(hipStreamSynchronize(s->stream));
+            if ((rc = step_once(s)) != 0 || (rc = settle(s)) != 0) return rc;
         const auto t0 = std::chrono::steady_clock::now();
-        if ((rc = step_once(s)) != 0) return rc;
-        HIPCHK(hipStreamSynchronize(s->stream));
+        if ((rc = step_once(s)) != 0 || (rc = settle(s)) != 0) return rc;
         *ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
         return 0;
     };
@@ -2064,7 +2075,7 @@ extern "C" int ecm_sim_get_neighbors(ecm_sim* s, int* nbr, int* cnt) {
     HIPCHK(launch_export_nbrs(d, dn.p, dc.p, s->stream));
     HIPCHK(hipMemcpyAsync(nbr, dn.p, N * s->prm.k * sizeof(int), hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipMemcpyAsync(cnt, dc.p, N * sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    if (int rc_ = settle(s)) return rc_;
     dn.release();
     dc.release();
     return 0;

@@ -331,6 +331,12 @@ class Simulator:
         N.check(self._L.ecm_sim_graph_status(self._h, C.byref(a), why, 512))
         return bool(a.value), why.value.decode()
 
+    def graph_counts(self):
+        """(steps that replayed a graph, graphs captured) since create."""
+        a, b = C.c_uint64(), C.c_uint64()
+        N.check(self._L.ecm_sim_graph_counts(self._h, C.byref(a), C.byref(b)))
+        return a.value, b.value
+
     def tuning(self) -> dict:
         t = N.SimTuning()
         N.check(self._L.ecm_sim_get_tuning(self._h, C.byref(t)))

@@ -70,10 +70,11 @@ int ecm_sim_log_step(ecm_sim* sim, ecm_mlp* m, int* n_logged);
 int ecm_mlp_train(ecm_mlp* m, int epochs, int batch, float lr, float pos_weight, float vel_weight, uint64_t seed,
                   float* losses);
 
-/* Forward pass of n host samples (x: n*64 FP32, rounded to BF16) with the inference kernel: y (n*16) raw outputs.  This call and
- * ecm_mlp_loss_grad stage the batch in 4 MiB of page-locked memory that the
- * handle makes at the first such call with more than 512 rows, or at the
- * second, and keeps: the call that makes it takes some 80 us more. */
+/* Forward pass of n host samples (x: n*64 FP32, rounded to BF16) with the
+ * inference kernel: y (n*16) raw outputs.  This call and ecm_mlp_loss_grad
+ * stage the batch in 4 MiB of page-locked memory that the handle makes at the
+ * first such call with more than 512 rows, or at the second, and keeps: the
+ * call that makes it takes some 80 us more. */
 int ecm_mlp_forward(ecm_mlp* m, const float* x, int n, float* y);
 
 /* ecm_mlp_forward for device buffers, allocating nothing: x (n*64 FP32)

@@ -112,6 +112,8 @@ int ecm_sim_set_replan_threads(ecm_sim* s, int n);
  * graphs are in use and, if not, why. */
 int ecm_sim_set_graph(ecm_sim* s, int on);
 int ecm_sim_graph_status(ecm_sim* s, int* active, char* why, int cap);
+/* Steps that replayed a graph and graphs captured, since create. */
+int ecm_sim_graph_counts(ecm_sim* s, uint64_t* replays, uint64_t* captures);
 
 /* Launch shape; no choice changes any result.  cell_scale multiplies the
  * agent grid cell edge (about one agent per cell at 1; default 1.25),

@@ -1,0 +1,44 @@
+"""How a step is put on the stream: with graphs on, a step that finds the
+stream idle replays its graph (the autotuner's samples among them, and a step
+behind one whose events overflowed the host block)."""
+import numpy as np
+import pytest
+
+from ecmgenerator_amd.simulator import Agents, Params, Simulator
+from helpers import small_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def walkers(n, seed, half=60.0, far=1000.0, extra=0):
+    """n agents on their way to goals far outside: none arrives."""
+    rng = np.random.default_rng(seed)
+    start = rng.uniform(-half, half, (n, 2)).astype(np.float32)
+    path = np.stack([start, start * 0 + np.float32(far)], 1).reshape(-1, 2).astype(np.float32)
+    agents = Agents(start, rng.uniform(0.2, 0.3, n).astype(np.float32), rng.uniform(1.0, 1.6, n).astype(np.float32),
+                    np.arange(n, dtype=np.int32) * 2, np.full(n, 2, np.int32), path)
+    box, _, obs, ecm, _ = small_scene(seed, half=half + 40.0, n_rects=3, n_agents=1, side=(1, 3))
+    sim = Simulator(ecm, obs, box, Params(max_agents=n + extra))
+    sim.SpawnAgents(agents, validate=False)
+    return sim, agents
+
+
+def test_autotune_times_graph_replays():
+    sim, _ = walkers(1500, 3)
+    sim.set_graph(True)
+    sim.Update()
+    steps, replays = sim.stats()["steps"], sim.graph_counts()[0]
+    sim.autotune(2)
+    assert sim.graph_counts()[0] - replays == sim.stats()["steps"] - steps > 20
+    sim.close()
+
+
+def test_step_behind_an_event_overflow_replays():
+    """2,000 agents outside every cell ask for a path each step: the step waits for the device's list."""
+    sim, agents = walkers(2000, 4, half=20.0)
+    sim.set_graph(True)
+    sim.write("position", np.full((2000, 2), 500.0, np.float32) + agents.start)
+    sim.Update(steps=4)
+    assert sim.replans().size == 2000
+    assert sim.graph_counts()[0] == 4
+    sim.close()
