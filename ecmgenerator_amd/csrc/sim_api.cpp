@@ -8,6 +8,7 @@
 #include "mlp_host.h"
 #include "sim_device.h"
 #include "replan_pool.h"
+#include "row_rule.h"
 
 #include <hip/hip_runtime.h>
 
@@ -281,8 +282,7 @@ struct ecm_sim {
     bool use_graph = false;
     bool idle = true;                           // no step queued on the stream since it was last waited for
     uint64_t graph_replays = 0, graph_captures = 0;
-    bool row_step = false, row_attr = false;    // 16 lanes per agent (row_rule)
-    int row_agents = 0;                         // agents their grid is sized for
+    RowRule row;                                // 16 lanes per agent
     StepGraph graphs[2][2];                     // [parity][entry from the sorted outputs]
     std::string graph_error;
     std::vector<int> h_replans;
@@ -1575,20 +1575,6 @@ static int prepare_step(ecm_sim* s, DevState* out) {
     return 0;
 }
 
-// 16 lanes per agent (row_kernels.h) for the plain step of a small crowd in
-// the default launch shape; other shapes say how agents are laid out.
-static constexpr int kRowAgents = 160000, kRowAttrAgents = 16000;
-
-static void row_rule(ecm_sim* s, int mode) {
-    // a crowd near a limit keeps the form it has: changing it captures the
-    // step graphs anew
-    auto small = [&](bool now, int limit) { return s->num_agents <= (now ? limit + limit / 4 : limit); };
-    const bool shape = mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2;
-    s->row_step = shape && small(s->row_step, kRowAgents);
-    s->row_attr = shape && small(s->row_attr, kRowAttrAgents);
-    s->row_agents = s->row_step ? (s->num_agents + 4095) / 4096 * 4096 : 0;
-}
-
 static int step_mode(const ecm_sim* s) { return s->log_mlp ? 1 : (s->mlp ? 2 : 0); }
 
 // The device operations of one step, in stream order, in two halves: up to
@@ -1602,11 +1588,11 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
         // events are final once the attraction pass is done: its last block
         // writes them to host memory, and the host handles them while the
         // neighbour search and the ORCA kernels run.
-        HIPCHK(launch_grid_attr(d, s->row_attr, s->n_cu, s->stream, s->timing ? s->ev[1] : nullptr));
+        HIPCHK(launch_grid_attr(d, s->row.attr, s->n_cu, s->stream, s->timing ? s->ev[1] : nullptr));
         if (s->timing) HIPCHK(hipEventRecord(s->ev[6], s->stream));
         // the plain step's main ORCA pass may run inside the k-nearest
         // kernel, or the whole rest of the step in one kernel
-        if (s->row_step) HIPCHK(launch_row_step(d, s->maxo, s->row_agents, s->stream));
+        if (s->row.step) HIPCHK(launch_row_step(d, s->maxo, s->row.agents, s->stream));
         else HIPCHK(launch_knn(d, s->tune.knn_block, mode, s->tune.orca_obst_slots, s->stream));
         return 0;
     }
@@ -1618,7 +1604,7 @@ static int enqueue_device_half(ecm_sim* s, const DevState& d, int mode, int half
                                      s->mlp_theta, s->mlp_mask.p, nullptr, nullptr, s->mlp->n_cu, s->stream));
     }
     if (s->timing) HIPCHK(hipEventRecord(s->ev[3], s->stream));
-    if (s->row_step) {
+    if (s->row.step) {
         if (s->timing) HIPCHK(hipEventRecord(s->ev[5], s->stream));
     } else {
         HIPCHK(launch_orca(d, s->maxo, mode, s->tune.orca_obst_slots, s->n_cu, s->stream,
@@ -1675,8 +1661,8 @@ static int ensure_step_graph(ecm_sim* s, const DevState& d, int mode) {
     key.frags = mode == 2 ? (const void*)s->mlp->frags.p : nullptr;
     key.pbias = mode == 2 ? (const void*)s->mlp->pbias.p : nullptr;
     key.n_cu = mode == 2 ? s->mlp->n_cu : 0;
-    key.row_agents = s->row_agents;
-    key.row = (s->row_step ? 1 : 0) | (s->row_attr ? 2 : 0);
+    key.row_agents = s->row.agents;
+    key.row = (s->row.step ? 1 : 0) | (s->row.attr ? 2 : 0);
     ecm_sim::StepGraph& g = s->graphs[s->cur][d.sorted_in];
     if (g.valid && std::memcmp(&g.key, &key, sizeof(key)) == 0) return 0;
     if (int rc = settle(s)) return rc;      // an earlier launch of g may still run
@@ -1716,7 +1702,7 @@ static int step_once(ecm_sim* s) {
     int rc = prepare_step(s, &d);
     if (rc) return rc;
     const int mode = step_mode(s);
-    row_rule(s, mode);
+    s->row.update(mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2, s->num_agents);
     // A step replays its graph when it finds the stream idle: one call then
     // puts all its kernels behind each other.  Behind a step that still runs
     // (a loop of steps with nothing read in between) its kernels are

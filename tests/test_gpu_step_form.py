@@ -1,6 +1,7 @@
 """How a step is put on the stream: with graphs on, a step that finds the
 stream idle replays its graph (the autotuner's samples among them, and a step
-behind one whose events overflowed the host block)."""
+behind one whose events overflowed the host block), and a crowd whose count
+moves around a multiple of 4,096 does not capture its graphs anew."""
 import numpy as np
 import pytest
 
@@ -41,4 +42,27 @@ def test_step_behind_an_event_overflow_replays():
     sim.Update(steps=4)
     assert sim.replans().size == 2000
     assert sim.graph_counts()[0] == 4
+    sim.close()
+
+
+def test_moving_count_keeps_the_graphs():
+    sim, agents = walkers(4100, 5, extra=8)
+    sim.set_graph(True)
+    ids = list(np.flatnonzero(sim.GetActiveFlags()))
+    one = Agents(agents.start[:1], agents.radius[:1], agents.pref_speed[:1], agents.path_off[:1], agents.path_cnt[:1],
+                 agents.path_xy[:2])
+    captures = 0
+    for it in range(12):                         # 4,100, then 4,090 and back, two steps each
+        if it % 4 == 2:
+            for i in ids[-10:]:
+                sim.DestroyAgent(int(i))
+            ids = ids[:-10]
+        elif it % 4 == 0 and it:
+            ids += [int(sim.SpawnAgents(one, validate=False)[0]) for _ in range(10)]
+        sim.Update()
+        sim.GetPositionData()
+        if it == 4:                              # both parities, entered from the slots and from the last step
+            captures = sim.graph_counts()[1]
+    assert sim.GetNumAgents() == 4090
+    assert sim.graph_counts() == (12, captures)
     sim.close()
