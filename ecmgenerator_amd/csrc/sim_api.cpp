@@ -1702,7 +1702,8 @@ static int step_once(ecm_sim* s) {
     int rc = prepare_step(s, &d);
     if (rc) return rc;
     const int mode = step_mode(s);
-    s->row.update(mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2, s->num_agents);
+    s->row.update(mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2, s->prm.k,
+                  s->num_agents);
     // A step replays its graph when it finds the stream idle: one call then
     // puts all its kernels behind each other.  Behind a step that still runs
     // (a loop of steps with nothing read in between) its kernels are
