@@ -262,7 +262,10 @@ struct ecm_sim {
     ecm_mlp* log_mlp = nullptr;     // set for the duration of ecm_sim_log_step
 
     // launch shape (results do not depend on it; ecm_sim_autotune picks it)
-    ecm_sim_tuning tune{1.25f, 256, 2, 0.0f};   // the shape the autotuner picks at 100k-2M agents
+    // the shape the autotuner picks at 100k-2M agents, and the one whose plain
+    // step may take 16 lanes per agent (row_rule.h)
+    static constexpr int kDefaultBlock = 256, kDefaultSlots = 2;
+    ecm_sim_tuning tune{1.25f, kDefaultBlock, kDefaultSlots, 0.0f};
     // the device part of a step captured as two hipGraphs (up to the replan
     // read-back, and the rest), one pair per position buffer parity,
     // recaptured when anything they were captured with changes
@@ -1702,8 +1705,9 @@ static int step_once(ecm_sim* s) {
     int rc = prepare_step(s, &d);
     if (rc) return rc;
     const int mode = step_mode(s);
-    s->row.update(mode == 0 && s->tune.knn_block == 256 && s->tune.orca_obst_slots == 2, s->prm.k,
-                  s->num_agents);
+    s->row.update(mode == 0 && s->tune.knn_block == ecm_sim::kDefaultBlock &&
+                      s->tune.orca_obst_slots == ecm_sim::kDefaultSlots,
+                  s->prm.k, s->num_agents);
     // A step replays its graph when it finds the stream idle: one call then
     // puts all its kernels behind each other.  Behind a step that still runs
     // (a loop of steps with nothing read in between) its kernels are
@@ -1868,10 +1872,12 @@ extern "C" int ecm_sim_set_tuning(ecm_sim* s, const ecm_sim_tuning* t) {
     return 0;
 }
 
-// Coordinate search over the launch shape on the live workload: the agent
-// grid cell scale, then the k-nearest block size, then the obstacle slots
-// of the main ORCA tile.  Every trial runs one untimed step (rebuilds) and
-// `steps` timed steps; the simulation advances through all of them.
+// Search over the launch shape on the live workload: the shape in use against
+// the default workgroup and slots, which together let the plain step of a
+// small crowd take 16 lanes per agent and which no change of one of them
+// reaches, then coordinate by coordinate the agent grid cell scale, the
+// k-nearest block size and the obstacle slots of the main ORCA tile.  The
+// simulation advances through all trials.
 extern "C" int ecm_sim_autotune(ecm_sim* s, int steps, ecm_sim_tuning* out) {
     if (!s || steps < 1) return fail(ECM_E_ARG, "bad autotune arguments");
     for (size_t e = 0; e < s->envs.size(); ++e)
@@ -1903,16 +1909,18 @@ extern "C" int ecm_sim_autotune(ecm_sim* s, int steps, ecm_sim_tuning* out) {
     const float scales[] = {0.6f, 0.8f, 1.0f, 1.25f, 1.6f, 2.0f};
     const int blocks[] = {64, 128, 256, 16};
     const int slots[] = {1, 2, 4};
-    for (int dim = 0; dim < 3; ++dim) {
+    for (int dim = -1; dim < 3; ++dim) {
         std::vector<ecm_sim_tuning> opts{best};
-        const int nopt = dim == 0 ? 6 : (dim == 1 ? 4 : 3);
+        const int nopt = dim < 0 ? 1 : (dim == 0 ? 6 : (dim == 1 ? 4 : 3));
         for (int o = 0; o < nopt; ++o) {
             ecm_sim_tuning t = best;
-            if (dim == 0) t.cell_scale = scales[o];
+            if (dim < 0) { t.knn_block = ecm_sim::kDefaultBlock; t.orca_obst_slots = ecm_sim::kDefaultSlots; }
+            else if (dim == 0) t.cell_scale = scales[o];
             else if (dim == 1) t.knn_block = blocks[o];
             else t.orca_obst_slots = slots[o];
             if (std::memcmp(&t, &best, sizeof(t)) != 0) opts.push_back(t);
         }
+        if (dim < 0 && opts.size() == 1) continue;
         std::vector<std::vector<float>> ms(opts.size());
         for (int r = 0; r < steps; ++r)
             for (size_t o = 0; o < opts.size(); ++o) {

@@ -138,8 +138,9 @@ typedef struct ecm_sim_tuning {
 } ecm_sim_tuning;
 int ecm_sim_get_tuning(ecm_sim* s, ecm_sim_tuning* out);
 int ecm_sim_set_tuning(ecm_sim* s, const ecm_sim_tuning* t);
-/* Coordinate search of the launch shape on the current workload: the
- * options of each coordinate are sampled round robin, `steps` rounds of one
+/* Search of the launch shape on the current workload: first the shape in use
+ * against the default knn_block and orca_obst_slots, then coordinate by
+ * coordinate.  The options are sampled round robin, `steps` rounds of one
  * timed step each (after two untimed ones), and compared by their median;
  * the simulation advances through every sampled step.  The best shape is
  * kept and returned. */

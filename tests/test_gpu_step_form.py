@@ -1,7 +1,8 @@
 """How a step is put on the stream: with graphs on, a step that finds the
 stream idle replays its graph (the autotuner's samples among them, and a step
 behind one whose events overflowed the host block), and a crowd whose count
-moves around a multiple of 4,096 does not capture its graphs anew."""
+moves around a multiple of 4,096 does not capture its graphs anew.  The
+autotuner finds the form with 16 lanes per agent from any launch shape."""
 import numpy as np
 import pytest
 
@@ -65,4 +66,16 @@ def test_moving_count_keeps_the_graphs():
             captures = sim.graph_counts()[1]
     assert sim.GetNumAgents() == 4090
     assert sim.graph_counts() == (12, captures)
+    sim.close()
+
+
+@pytest.mark.parametrize("shape", [(64, 1), (16, 4), (128, 2), (256, 2)])
+def test_autotune_finds_the_row_step(shape):
+    """500 agents, three times as fast with 16 lanes each."""
+    sim, _ = walkers(500, 6)
+    sim.set_graph(True)
+    sim.set_tuning(knn_block=shape[0], orca_obst_slots=shape[1])
+    sim.Update()
+    t = sim.autotune(3)
+    assert (t["knn_block"], t["orca_obst_slots"]) == (256, 2)
     sim.close()
