@@ -2,17 +2,20 @@
 stream idle replays its graph (the autotuner's samples among them, and a step
 behind one whose events overflowed the host block), and a crowd whose count
 moves around a multiple of 4,096 does not capture its graphs anew.  The
-autotuner finds the form with 16 lanes per agent from any launch shape."""
+autotuner finds the form with 16 lanes per agent from any launch shape, and a
+crowd that crosses the form's limits gives the same steps as one that never
+takes it."""
 import numpy as np
 import pytest
 
 from ecmgenerator_amd.simulator import Agents, Params, Simulator
 from helpers import small_scene
+from test_gpu_row_step import same
 
 pytestmark = pytest.mark.gpu
 
 
-def walkers(n, seed, half=60.0, far=1000.0, extra=0):
+def walkers(n, seed, half=60.0, far=1000.0, extra=0, k=10, keep=False):
     """n agents on their way to goals far outside: none arrives."""
     rng = np.random.default_rng(seed)
     start = rng.uniform(-half, half, (n, 2)).astype(np.float32)
@@ -20,7 +23,7 @@ def walkers(n, seed, half=60.0, far=1000.0, extra=0):
     agents = Agents(start, rng.uniform(0.2, 0.3, n).astype(np.float32), rng.uniform(1.0, 1.6, n).astype(np.float32),
                     np.arange(n, dtype=np.int32) * 2, np.full(n, 2, np.int32), path)
     box, _, obs, ecm, _ = small_scene(seed, half=half + 40.0, n_rects=3, n_agents=1, side=(1, 3))
-    sim = Simulator(ecm, obs, box, Params(max_agents=n + extra))
+    sim = Simulator(ecm, obs, box, Params(max_agents=n + extra, k=k, keep_orca_velocity=keep))
     sim.SpawnAgents(agents, validate=False)
     return sim, agents
 
@@ -79,3 +82,32 @@ def test_autotune_finds_the_row_step(shape):
     t = sim.autotune(3)
     assert (t["knn_block"], t["orca_obst_slots"]) == (256, 2)
     sim.close()
+
+
+@pytest.mark.parametrize("limit,k", [(112000, 5), (16000, 10)])
+def test_crossing_a_limit(limit, k):
+    """The step's limit at k 5 and the attraction pass's: past it, an eighth below it and past it again, with graphs."""
+    n, back = limit - 10, limit - limit // 8 - 10
+    sims = []
+    for shape in (256, 64):
+        sim, agents = walkers(n, 8, half=float(np.sqrt(n / 0.3) / 2), extra=limit // 8 + 100, k=k, keep=True)
+        sim.set_tuning(knn_block=shape)
+        sim.set_graph(True)
+        sims.append(sim)
+
+    def part(m):
+        return Agents(agents.start[:m] + np.float32(0.4), agents.radius[:m], agents.pref_speed[:m], agents.path_off[:m],
+                      agents.path_cnt[:m], agents.path_xy)
+    for act in ("", "", "over", "", "below", "", "over", ""):
+        for sim in sims:
+            have = sim.GetNumAgents()
+            if act == "over":
+                sim.SpawnAgents(part(limit + 20 - have), validate=False)
+            elif act == "below":
+                for i in np.flatnonzero(sim.GetActiveFlags())[:have - back]:
+                    sim.DestroyAgent(int(i))
+            sim.Update()
+        assert sims[0].GetNumAgents() in (n, limit + 20, back)
+        same(*sims)
+    for sim in sims:
+        sim.close()
