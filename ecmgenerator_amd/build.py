@@ -80,6 +80,14 @@ def build(verbose: bool = True) -> str:
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"facade driver build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    # the device code's own arithmetic, checked against plain operations by a GPU test
+    chk = os.path.join(HERE, "..", "tests", "cpp", "arith_check.hip")
+    if os.path.exists(chk):
+        out = os.path.join(HERE, "..", "tests", "cpp", "_build", "libarith_check.so")
+        cmd = [HIPCC] + COMMON + ["-shared", "-I", CSRC, chk, "-o", out]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"arithmetic check build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     if verbose:
         print(f"built {LIB}", file=sys.stderr)
     return LIB

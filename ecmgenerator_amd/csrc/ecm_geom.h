@@ -221,11 +221,11 @@ ECM_HD void rotate_pm(V2 v, float rad, V2& plus, V2& minus) {
 // 1 / l gives it correctly rounded; and with that, q = n y corrected by its
 // exact residual is the correctly rounded n / l (Markstein, "Computation of
 // elementary functions on the IBM RISC System/6000 processor", 1990).
-// Checked on gfx950 without an exception: the root for every S in [2^-100,
-// 2^100], the reciprocal from rcp for every mantissa and every exponent in
-// [-60, 60), the quotient for every pair of 23-bit mantissas.  The
-// reciprocal from rsq is correct for every l but the one of all-ones
-// mantissa.  In a loop of 8 waves per SIMD a wavefront takes 18.3 ns for `/`,
+// Checked on gfx950 without an exception (tests/cpp/arith_check.hip): the root
+// for every S in [2^-96, 2^96), the reciprocal from rcp, and that from rsq for
+// every l but the one of all-ones mantissa, for every mantissa and exponent
+// they are used at, 2^28 quotients over the whole range, their extreme
+// mantissas among them, and the arc tangent of every float in [0, 1].  In a loop of 8 waves per SIMD a wavefront takes 18.3 ns for `/`,
 // 21.4 for sqrtf, 60.7 for two components over their length; here 13.5, 12.5
 // and 31.
 constexpr uint32_t kExp = 1u << 23;
@@ -250,7 +250,8 @@ __device__ __forceinline__ float recip_from(float l, float y) {
     return __builtin_fmaf(__builtin_fmaf(-l, y, 1.0f), y, y);
 }
 // n / l for l > 0 and y its correctly rounded reciprocal, both in [2^-60,
-// 2^60), n zero or in [2^-80, 2^60) in magnitude.  The residual is taken
+// 2^60), n zero or in [2^-80, 2^60) in magnitude, where the quotient is a
+// normal number (no kernel forms one below 2^-112).  The residual is taken
 // negated: for n = -0 it is then +0, and the quotient -0.
 __device__ __forceinline__ float quot(float n, float l, float y) {
     const float q = n * y;
