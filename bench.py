@@ -170,6 +170,7 @@ def main():
     for _ in range(n_kt):
         sim.Update()
         kt += np.array(sim.last_timing())
+    row_step = sim.last_step_row()
     sim.set_timing(False)
     updates = st1["agent_updates"] - st0["agent_updates"]
     # beside (never as) the value: the rate when every step is followed by
@@ -196,14 +197,7 @@ def main():
     # phases (HIP events on the simulator's stream; no proposal phase in the
     # plain step), one kernel each except the grid build and the queue passes
     shape = sim.get_tuning()
-    fused = wl.params.k in (5, 10) and shape["orca_obst_slots"] == 2
-    phases = {"grid_build": kt[0], "attraction": kt[5]}
-    if fused:           # k_knn_orca: the k-nearest pass and the main ORCA pass in one kernel
-        phases["knn_orca_main"] = kt[1] - kt[5]
-    else:
-        phases["knn"] = kt[1] - kt[5]
-        phases["orca_main"] = kt[4]
-    phases["orca_queues"] = kt[3] - kt[4]
+    phases = plain_phases(kt, wl.params.k, shape["orca_obst_slots"], row_step)
     # the roofline is quoted on the longest single kernel
     singles = [k for k in phases if k not in ("grid_build", "orca_queues")]
     dom_name = max(singles, key=lambda k: phases[k])
@@ -217,20 +211,7 @@ def main():
     b_agent = 58.0 + 8.0 * mean_path
     achieved = b_agent * n_per_step / (dom_ms * 1e-3) / 1e9
     # each kernel's own minimum state traffic per agent, for comparison
-    k = wl.params.k
-    own_bytes = {
-        "grid_build": 1 + 8 + 8 + 4 + 4 + 4 + 16 + 8 + 4,
-        # state 16 + 8, path offset and count 8, path points 8 P, attraction
-        # point read and written 16, preferred velocity 8, destroyed flag 1
-        "attraction": 16 + 8 + 8 + 8 * mean_path + 16 + 8 + 1,
-        # state 16, seeds (previous list 4 k + count 4 + map 4), list and count written 4 k + 4
-        "knn": 16 + 4 * k + 4 + 4 + 4 * k + 4,
-        # state 16 + 8, destroyed flag, radius 4, preferred velocity 8, list
-        # and count 4 k + 4, position and velocity written 8 + 8
-        "orca_main": 16 + 8 + 1 + 4 + 8 + 4 + 4 * k + 8 + 8,
-    }
-    # the kernel running both reads the state, the list and its count once
-    own_bytes["knn_orca_main"] = own_bytes["knn"] + own_bytes["orca_main"] - (16 + 4 * k + 4)
+    own_bytes = own_bytes_per_agent(wl.params.k, mean_path)
     traffic, tsrc = _profiled(name, dom_name, "traffic")
     valu, _ = _profiled(name, dom_name, "valu_busy")
     step_gbs = b_agent * n_per_step / (ms_per_step * 1e-3) / 1e9
@@ -286,6 +267,46 @@ def main():
         "stats": {k: st1[k] - st0[k] for k in st1},
     }
     print(json.dumps(line), flush=True)
+
+
+def plain_phases(kt, k, obst_slots, row_step):
+    """The plain step's phases in ms from the six timings (ecm_sim_last_timing):
+    one kernel each except the grid build (count and prefix sum) and the queue
+    passes.  "attraction" is the sort of the agents into the grid and the
+    attraction pass, one kernel."""
+    phases = {"grid_build": kt[0], "attraction": kt[5]}
+    if row_step:                                     # k_row_step: the whole rest of the step
+        phases["row_step"] = kt[1] - kt[5]
+        return phases
+    if k in (5, 10) and obst_slots == 2:             # k_knn_orca: the k-nearest and the main ORCA pass
+        phases["knn_orca_main"] = kt[1] - kt[5]
+    else:
+        phases["knn"] = kt[1] - kt[5]
+        phases["orca_main"] = kt[4]
+    phases["orca_queues"] = kt[3] - kt[4]
+    return phases
+
+
+def own_bytes_per_agent(k, mean_path):
+    """Each phase's own minimum state traffic per agent."""
+    own = {
+        # position 8 and destroyed flag 1 read; key and rank written 4 + 4
+        "grid_build": 8 + 1 + 4 + 4,
+        # sort: key, rank and cell start 4 each, position, velocity, radius and
+        # id, speed and environment, attraction point, path offset and count 8
+        # each; the sorted state 16 + 16, path 8 and the maps between the two
+        # orders 4 + 4 written.  Attraction: path points 8 P; attraction point
+        # 8, preferred velocity 8, destroyed flag 1 written
+        "attraction": 3 * 4 + 6 * 8 + 16 + 16 + 8 + 4 + 4 + 8 * mean_path + 8 + 8 + 1,
+        # state 16, seeds (previous list 4 k + count 4 + map 4), list and count written 4 k + 4
+        "knn": 16 + 4 * k + 4 + 4 + 4 * k + 4,
+        # state 16 + 8, destroyed flag, radius 4, preferred velocity 8, list
+        # and count 4 k + 4, position and velocity written 8 + 8
+        "orca_main": 16 + 8 + 1 + 4 + 8 + 4 + 4 * k + 8 + 8,
+    }
+    # a kernel running both reads the state, the list and its count once
+    own["knn_orca_main"] = own["row_step"] = own["knn"] + own["orca_main"] - (16 + 4 * k + 4)
+    return own
 
 
 def _profiled(workload, kernel, what):

@@ -252,7 +252,7 @@ struct ecm_sim {
     bool timing = false;
     // [5]: after the main ORCA pass, [6]: after the attraction pass
     hipEvent_t ev[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    float last_ms[6] = {0, 0, 0, 0, 0, 0};
+    float last_ms[7] = {0, 0, 0, 0, 0, 0, 0};
 
     // learned proposal (features + network + verification) and sample log
     ecm_mlp* mlp = nullptr;
@@ -1797,6 +1797,7 @@ static int step_once(ecm_sim* s) {
         s->last_ms[4] = ms;
         HIPCHK(hipEventElapsedTime(&ms, s->ev[1], s->ev[6]));
         s->last_ms[5] = ms;
+        s->last_ms[6] = s->row.step ? 1.0f : 0.0f;
     }
     return 0;
 }
@@ -2135,7 +2136,7 @@ extern "C" int ecm_sim_set_timing(ecm_sim* s, int on) {
 }
 extern "C" int ecm_sim_last_timing(ecm_sim* s, float* out, int n) {
     if (!s || !out || n < 0) return fail(ECM_E_ARG, "null argument");
-    for (int i = 0; i < n && i < 6; ++i) out[i] = s->last_ms[i];
+    for (int i = 0; i < n && i < 7; ++i) out[i] = s->last_ms[i];
     return 0;
 }
 

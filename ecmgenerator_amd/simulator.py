@@ -313,12 +313,20 @@ class Simulator:
         N.check(self._L.ecm_sim_set_timing(self._h, int(on)))
 
     def last_timing(self):
-        """[grid build, attraction + k-nearest, learned proposal, ORCA + LP +
-        integration, the main ORCA pass alone, the attraction pass alone]
-        device ms of the last step (with set_timing(True))."""
+        """[counting and prefix sum of the grid build, sort + attraction +
+        k-nearest, learned proposal, ORCA + LP + integration, the main ORCA
+        pass alone, the sort and attraction pass alone] device ms of the last
+        step (with set_timing(True)).  With 16 lanes per agent the second
+        holds the ORCA passes too (last_step_row)."""
         a = (C.c_float * 6)()
         N.check(self._L.ecm_sim_last_timing(self._h, a, 6))
         return list(a)
+
+    def last_step_row(self) -> bool:
+        """Whether the last timed step took 16 lanes per agent."""
+        a = (C.c_float * 7)()
+        N.check(self._L.ecm_sim_last_timing(self._h, a, 7))
+        return a[6] != 0.0
 
     def set_graph(self, on: bool = True) -> None:
         """Replay the device part of each step as captured hipGraphs."""

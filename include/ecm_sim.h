@@ -119,17 +119,20 @@ int ecm_sim_graph_counts(ecm_sim* s, uint64_t* replays, uint64_t* captures);
  * agent grid cell edge (about one agent per cell at 1; default 1.25),
  * knn_block is the workgroup size of the k-nearest kernel (64,
  * 128, 256; default 256; 16: 16 agents per 64-lane wavefront of the fused
- * kernel below, for crowds of a few thousand agents, and 64 otherwise),
- * and orca_obst_slots sizes the main ORCA pass (1,
- * 2, 4; default 2): the plain step holds 4 obstacle constraints per agent
- * in registers (8 with orca_obst_slots 4 and k <= 10) and sends agents with
- * more to the overflow pass; with orca_obst_slots 2 and k 5 or 10 that pass
- * runs inside the k-nearest kernel; the learned and logging steps
+ * kernel below, and 64 otherwise), and orca_obst_slots sizes the main ORCA
+ * pass (1, 2, 4; default 2): the plain step holds 4 obstacle constraints per
+ * agent in registers (8 with orca_obst_slots 4 and k <= 10) and sends agents
+ * with more to the overflow pass; with orca_obst_slots 2 and k 5 or 10 that
+ * pass runs inside the k-nearest kernel, whose workgroups are 64 threads for
+ * knn_block 256 too; the learned and logging steps
  * give each agent orca_obst_slots slots beyond k in an LDS tile, agents
  * with more constraints borrow from their workgroup's small spill area, and
  * those with more obstacle constraints than the tile holds, or whose
- * workgroup's spill area is used up, take the overflow pass.  best_ms: step
- * time the autotuner measured (0 before). */
+ * workgroup's spill area is used up, take the overflow pass.  The default pair
+ * (256, 2) also lets the plain step of a small crowd (up to 112,000 agents at
+ * k <= 5, 160,000 at k <= 10, 200,000 above) take 16 lanes per agent, two to
+ * four times as fast for a few thousand agents as any other shape.  best_ms:
+ * step time the autotuner measured (0 before). */
 typedef struct ecm_sim_tuning {
     float cell_scale;
     int knn_block;
@@ -228,14 +231,19 @@ int ecm_sim_get_replans(ecm_sim* s, int* ids, int cap, int* n);
 #define ECM_SIM_N_STATS 11
 int ecm_sim_stats(ecm_sim* s, uint64_t* out, int n);
 /* Device time of the phases of the last step in ms (HIP events on the
- * handle's stream): [0] grid build, [1] attraction + k-nearest, [2] learned
+ * handle's stream): [0] the grid build's counting and prefix sum, [1] the
+ * sort of the agents into the grid, attraction and k-nearest, [2] learned
  * proposal (features + network; 0 without one), [3] ORCA + LP +
  * integration, [4] of [3], the main ORCA pass alone (the rest is the
  * passes over its queues: obstacle overflow and the 3D LP), [5] of [1], the
- * attraction pass alone (goal checks, IRM, steering; the rest is the
- * k-nearest pass).  In the plain step with k 5 or 10 and orca_obst_slots 2
- * the main ORCA pass runs inside the k-nearest kernel: [1] includes it and
- * [4] is empty.  Enable with ecm_sim_set_timing(s, 1); copies min(n, 6). */
+ * sort and the attraction pass (goal checks, IRM, steering), one kernel except
+ * after a step that reads the slot arrays, where the sort is in [0]; the rest
+ * is the k-nearest pass.  In the plain step with k 5 or 10 and orca_obst_slots
+ * 2 the main ORCA pass runs inside the k-nearest kernel: [1] includes it and
+ * [4] is empty.  With 16 lanes per agent (small crowds in the default launch
+ * shape, see ecm_sim_tuning) the whole rest of the step does: [1] includes it,
+ * [3] and [4] are empty, and [6] is 1, else 0.  Enable with
+ * ecm_sim_set_timing(s, 1); copies min(n, 7). */
 int ecm_sim_set_timing(ecm_sim* s, int on);
 int ecm_sim_last_timing(ecm_sim* s, float* out, int n);
 

@@ -111,3 +111,15 @@ def test_crossing_a_limit(limit, k):
         same(*sims)
     for sim in sims:
         sim.close()
+
+
+def test_timing_names_the_form():
+    sim, _ = walkers(300, 9)
+    sim.set_timing(True)
+    for shape, row in (((256, 2), True), ((64, 2), False), ((256, 1), False), ((256, 2), True)):
+        sim.set_tuning(knn_block=shape[0], orca_obst_slots=shape[1])
+        sim.Update()
+        t = sim.last_timing()
+        assert sim.last_step_row() == row and len(t) == 6
+        assert t[1] >= t[5] > 0.0
+    sim.close()
