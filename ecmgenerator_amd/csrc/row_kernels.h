@@ -1,8 +1,8 @@
 // row_kernels.h -- the plain step's per-agent passes with 16 lanes per agent,
-// for crowds that leave most of the chip idle at one agent per lane.
-// Included by sim_kernels.hip inside namespace ecm.
+// for crowds that leave the chip idle at one agent per lane; row_rule.h says
+// up to which size.  Included by sim_kernels.hip inside namespace ecm.
 //
-// At one agent per lane, a crowd of 500 to 40,000 agents fills at most one
+// At one agent per lane, a crowd of up to some 65,000 agents fills at most one
 // wavefront per SIMD, and a pass lasts as long as one wavefront's chain of
 // dependent loads and unrolled code: 82-85 us for the neighbour search and
 // ORCA at 500 agents as at 5,000 (k 10), plus the queue kernels of the

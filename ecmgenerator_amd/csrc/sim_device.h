@@ -141,13 +141,13 @@ struct DevState {
                               // (their count in acc[15], cleared by the last attraction block)
 
     // ---- events ----
-    // One list per step, read back by the host after the neighbour pass:
-    // (id, x bits, y bits, 0) asks UpdatePath from the step-start position
-    // (x, y); (id, 0, 0, 1) is a DestroyAgent.
+    // One list per step, published by the attraction pass: (id, x bits, y
+    // bits, t >= 0) asks UpdatePath for the agent at sorted position t from the
+    // step-start position (x, y); (id, 0, 0, -1) is a DestroyAgent.
     int4* events;         uint32_t* events_n;
     uint32_t* stats;      // per step: [0] unused, [1] obstacle-overflow queue
                           // length, [2] locate fallbacks to the exact-y list, [3] blocks of
-                          // k_attr done, [4] 3D-LP entries with more obstacle constraints
+                          // the attraction pass done, [4] 3D-LP entries with more obstacle constraints
                           // than the register tile holds, [5] unused
     uint32_t* wstats;     // per step: the spread counters, [kStatSlots][kStatStride]
     uint32_t* group_done; // [kDoneGroups][kStatStride] blocks of the attraction pass finished, by group

@@ -4,7 +4,8 @@
 // Step pipeline (all on the handle's stream, no host round trip):
 //   1. k_grid_count / scan / k_grid_scatter: counting sort of the active
 //      agents by Morton cell (replaces KDTree::Construct, KDTree.cpp:22-83).
-//   2. k_attr: goal checks + IRM attraction point on the ECM
+//   2. k_scatter_attr (k_attr after a sort from the slot arrays): goal checks +
+//      IRM attraction point on the ECM
 //      (Simulator.cpp:538-590, IRMPathFollower.cpp:14-115, ECM.cpp:20-96,
 //      ECMCellCollection.cpp:57-90) and steering (Simulator.cpp:638-657); its
 //      last block publishes the step's replan and destroy events.
@@ -2294,7 +2295,12 @@ static void launch_orca_k(const DevState& s, int maxo, int mode, int oslots, int
 
 // The neighbour search and ORCA with 16 lanes per agent (row_kernels.h): the
 // rest of the plain step.  A wavefront for every four of `agents` (the kernel
-// strides, so that any count is covered).
+// strides, so that any count is covered).  Every wavefront has LDS for the
+// longest obstacle list, which past some 112 edges holds fewer of them on a CU
+// than the registers do; the one-lane passes lose more to such lists (20 steps
+// of 155,000 agents with a spot of 464 edges on their map: 6.5 ms here, 12.2
+// there; 110,000: 4.0 and 12.4; 40,000 between pillars 1.5 m apart: 5.1 and
+// 27.5).
 hipError_t launch_row_step(const DevState& s, int maxo, int agents, hipStream_t st) {
     const int row_f4 = std::max(maxo + kRow, kRowLdsBytes / 16);
     hipLaunchKernelGGL(k_row_step, dim3(round8(cdiv(std::max(1, std::min(agents, s.n_slots)), 4))), dim3(64),
