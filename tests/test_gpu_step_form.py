@@ -3,12 +3,13 @@ stream idle replays its graph (the autotuner's samples among them, and a step
 behind one whose events overflowed the host block), and a crowd whose count
 moves around a multiple of 4,096 does not capture its graphs anew.  The
 autotuner finds the form with 16 lanes per agent from any launch shape, and a
-crowd that crosses the form's limits gives the same steps as one that never
-takes it."""
+crowd that crosses the form's limits, or whose map has long obstacle lists,
+gives the same steps as one that never takes it."""
 import numpy as np
 import pytest
 
-from ecmgenerator_amd.simulator import Agents, Params, Simulator
+from ecmgenerator_amd import scenarios as S
+from ecmgenerator_amd.simulator import Agents, Obstacles, Params, Simulator
 from helpers import small_scene
 from test_gpu_row_step import same
 
@@ -123,3 +124,32 @@ def test_timing_names_the_form():
         assert sim.last_step_row() == row and len(t) == 6
         assert t[1] >= t[5] > 0.0
     sim.close()
+
+
+def test_long_obstacle_lists_in_a_large_crowd():
+    """30,000 agents and a spot of pillars with several hundred edges within range of one point: every wavefront of
+    the row step holds room for the longest list."""
+    n, half = 30000, 200.0
+    rng = np.random.default_rng(10)
+    start = rng.uniform(-half, half, (n, 2)).astype(np.float32)
+    start[:3000] = rng.uniform(-8.0, 8.0, (3000, 2))
+    goal = rng.uniform(-half, half, (n, 2)).astype(np.float32)
+    agents = Agents(start, rng.uniform(0.15, 0.25, n).astype(np.float32), rng.uniform(1.0, 1.6, n).astype(np.float32),
+                    np.arange(n, dtype=np.int32) * 2, np.full(n, 2, np.int32), np.stack([start, goal], 1).reshape(-1, 2))
+    c = (np.arange(9) - 4) * 1.0
+    rings = [S.rect_ring(x, y, 0.2, 0.2) for x in c for y in c]
+    obs = Obstacles(np.concatenate(rings).astype(np.float32), np.arange(len(rings) + 1, dtype=np.int32) * 4)
+    box = (-half - 5.0, -half - 5.0, half + 5.0, half + 5.0)
+    sims = []
+    for shape in (256, 64):
+        sim = Simulator(S.empty_square_ecm(*box), obs, box, Params(max_agents=n, keep_orca_velocity=True))
+        sim.SpawnAgents(agents, validate=False)
+        sim.set_tuning(knn_block=shape)
+        sims.append(sim)
+    for _ in range(4):
+        for sim in sims:
+            sim.Update()
+        same(*sims)
+    assert sims[0].stats()["lp3d_big"] > 100
+    for sim in sims:
+        sim.close()
